@@ -255,7 +255,7 @@ int gemv_group(const qk_weight* const* ws, void* const* ys, int cnt, bool glu, A
             if (rc != QK_OK || info) return rc;
             continue;
         }
-        // consecutive matrices of equal type share one launch; F32 matrices run one by one
+        // consecutive matrices of equal type share one launch
         for (int i = 0; i < cnt;) {
             if (ws[i]->type == QK_T_F32) {
                 if (info) {
@@ -264,10 +264,14 @@ int gemv_group(const qk_weight* const* ws, void* const* ys, int cnt, bool glu, A
                     info->token_slots = mt;
                     return QK_OK;
                 }
-                if (qk::launch_f32((const float*)ws[i]->data, k, ws[i]->n, xt.p, xt.fmt, mt,
-                                   (float*)out_at(ys[i], QK_ACT_F32, (size_t)t0 * ws[i]->n), s))
-                    return QK_E_HIP;
-                i++;
+                qk::F32Mats M{};
+                int c = 0;
+                for (; i < cnt && ws[i]->type == QK_T_F32; i++, c++) {
+                    M.w[c] = (const float*)ws[i]->data;
+                    M.n[c] = ws[i]->n;
+                    M.y[c] = (float*)out_at(ys[i], QK_ACT_F32, (size_t)t0 * ws[i]->n);
+                }
+                if (qk::launch_f32(M, c, k, xt.p, xt.fmt, mt, s)) return QK_E_HIP;
                 continue;
             }
             int j = i + 1;
@@ -338,8 +342,13 @@ int check_group(const qk_weight* const* ws, void* const* ys, int cnt, int glu, c
 
 // qk_matmul_act on the workspace wsp.
 int matmul_on(const qk_weight* w, Act x, int m, float* y, hipStream_t s, const Workspace* wsp) {
-    if (w->type == QK_T_F32)
-        return qk::launch_f32((const float*)w->data, w->k, w->n, x.p, x.fmt, m, y, s) ? QK_E_HIP : QK_OK;
+    if (w->type == QK_T_F32) {
+        qk::F32Mats M{};
+        M.w[0] = (const float*)w->data;
+        M.n[0] = w->n;
+        M.y[0] = y;
+        return qk::launch_f32(M, 1, w->k, x.p, x.fmt, m, s) ? QK_E_HIP : QK_OK;
+    }
     if (m >= gemm_route_m()) return run_gemm(w, x, m, y, s, wsp);
     const qk_weight* ws[1] = {w};
     void* ys[1] = {y};

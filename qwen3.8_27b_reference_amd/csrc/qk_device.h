@@ -234,6 +234,17 @@ __device__ inline float sum4(float v) { v = sum2(v); return v + dpp_xor2(v); }
 __device__ inline float sum8(float v) { v = sum4(v); return v + dpp_mirror8(v); }
 __device__ inline float sum16(float v) { v = sum8(v); return v + dpp_mirror16(v); }
 
+// Cross-row exchanges without the LDS: permlane16/32_swap(x, x) return the two halves whose sum
+// (or max) is the xor-16 (xor-32) reduction in every lane.
+__device__ inline float xor16_sum(float v) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), false, false);
+    return __builtin_bit_cast(float, (int)p[0]) + __builtin_bit_cast(float, (int)p[1]);
+}
+__device__ inline float xor32_sum(float v) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), false, false);
+    return __builtin_bit_cast(float, (int)p[0]) + __builtin_bit_cast(float, (int)p[1]);
+}
+
 __device__ inline u4 ld16(const void* p) { return *(const u4*)p; }
 __device__ inline u2 ld8(const void* p) { return *(const u2*)p; }
 __device__ inline uint32_t ld4(const void* p) { return *(const uint32_t*)p; }

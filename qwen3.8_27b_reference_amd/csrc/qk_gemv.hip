@@ -770,16 +770,6 @@ __device__ inline int a8_offset(int lane, int p) {
     return live ? (kg * MT * XP + i) * 16 : 64 * XP * MT;
 }
 
-// Cross-row exchanges without the LDS: permlane16/32_swap(x, x) return the two halves whose sum
-// (or max) is the xor-16 (xor-32) reduction in every lane.
-__device__ inline float xor16_sum(float v) {
-    const auto p = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), false, false);
-    return __builtin_bit_cast(float, (int)p[0]) + __builtin_bit_cast(float, (int)p[1]);
-}
-__device__ inline float xor32_sum(float v) {
-    const auto p = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), false, false);
-    return __builtin_bit_cast(float, (int)p[0]) + __builtin_bit_cast(float, (int)p[1]);
-}
 __device__ inline uint32_t xor16_umax(uint32_t v) {
     const auto p = __builtin_amdgcn_permlane16_swap((int)v, (int)v, false, false);
     return max((uint32_t)p[0], (uint32_t)p[1]);

@@ -121,9 +121,14 @@ void gemm_set_map(int map);  // tuning: 1 = one token block per XCD (default), 0
 bool gemm_set_pairs(int p);  // tuning override of the tile pairs per work-group (0 = planned)
 bool gemm_set_ksplit(int ks);  // tuning override of the K-parts (0 = planned, 1..16)
 
-// F32 weights, row-major [n][k] (GGUF layout): y[m][n] = x[m][k] W^T, fp32 accumulate, any m; x in
-// xfmt (ACT_*).
-int launch_f32(const float* w, int k, int n, const void* x, int xfmt, int m, float* y, hipStream_t s);
+// F32 weights, row-major [n][k] (GGUF layout): y[z][m][n[z]] = x[m][k] W[z]^T for cnt (1..4) matrices that
+// share x, in one launch; fp32 products and sums, any m, no workspace; x in xfmt (ACT_*).
+struct F32Mats {
+    const float* w[GEMV_MAX_CNT];
+    float* y[GEMV_MAX_CNT];
+    int n[GEMV_MAX_CNT];
+};
+int launch_f32(const F32Mats& mats, int cnt, int k, const void* x, int xfmt, int m, hipStream_t s);
 
 int launch_repack(const uint8_t* src, uint8_t* dst, int type, int k, int n, uint64_t rb, int dir, hipStream_t s);
 int launch_dequant(const uint8_t* w, int type, int layout, int k, int n, uint64_t rb, const int32_t* rows, int nrows,
