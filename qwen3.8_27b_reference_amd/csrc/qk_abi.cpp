@@ -471,7 +471,7 @@ int qk_repack(const qk_weight* src, void* dst, uint32_t dst_layout, qk_stream_t 
             return QK_E_HIP;
     } else {
         const int dir = dst_layout == QK_LAYOUT_T16 ? 0 : 1;
-        if (qk::launch_repack((const uint8_t*)src->data, (uint8_t*)dst, (int)src->type, src->k, src->n, src->rb, dir,
+        if (qk::launch_repack((const uint8_t*)src->data, (uint8_t*)dst, (int)src->type, src->k, src->n, dir,
                               (hipStream_t)stream) != 0)
             return QK_E_HIP;
     }
@@ -512,7 +512,7 @@ int qk_upload(const void* host, uint32_t type, int32_t k, int32_t n, uint32_t la
             return QK_E_HIP;
         }
         bool ok = hipMemcpyAsync(tmp, host, bytes, hipMemcpyHostToDevice, s) == hipSuccess &&
-                  qk::launch_repack((const uint8_t*)tmp, (uint8_t*)dst, (int)type, k, n, rb, 0, s) == 0 &&
+                  qk::launch_repack((const uint8_t*)tmp, (uint8_t*)dst, (int)type, k, n, 0, s) == 0 &&
                   hipStreamSynchronize(s) == hipSuccess;
         (void)hipFree(tmp);
         if (!ok) {

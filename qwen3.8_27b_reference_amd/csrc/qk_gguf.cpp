@@ -133,7 +133,7 @@ int read_file(const char* path, std::vector<uint8_t>& buf) {
 bool repackable(const qk_gguf::Tensor& t) {
     const bool quant = t.type == QK_T_Q8_0 || t.type == QK_T_Q4_K || t.type == QK_T_Q5_K || t.type == QK_T_Q6_K;
     return quant && t.ndims == 2 && t.dims[0] % 256 == 0 && t.dims[1] % 16 == 0 && t.dims[0] <= INT32_MAX &&
-           t.dims[1] <= INT32_MAX;
+           t.dims[1] <= INT32_MAX && t.offset % 16 == 0;  // a view of any other offset is refused (QK_E_ALIGN)
 }
 
 }  // namespace
@@ -276,10 +276,8 @@ int qk_gguf_upload(qk_gguf* f, qk_stream_t stream) {
         if (rc != QK_OK) break;
         if (!repackable(t)) continue;
         uint8_t* at = dev + t.offset;
-        uint64_t rb = 0;
-        (void)qk_row_bytes(t.type, t.dims[0], &rb);
         if (hipMemcpyAsync(scratch, at, t.nbytes, hipMemcpyDeviceToDevice, s) != hipSuccess ||
-            qk::launch_repack(scratch, at, (int)t.type, (int)t.dims[0], (int)t.dims[1], rb, 0, s) != 0)
+            qk::launch_repack(scratch, at, (int)t.type, (int)t.dims[0], (int)t.dims[1], 0, s) != 0)
             rc = QK_E_HIP;
     }
     if (hipStreamSynchronize(s) != hipSuccess && rc == QK_OK) rc = QK_E_HIP;

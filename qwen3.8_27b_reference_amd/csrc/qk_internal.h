@@ -130,7 +130,7 @@ struct F32Mats {
 };
 int launch_f32(const F32Mats& mats, int cnt, int k, const void* x, int xfmt, int m, hipStream_t s);
 
-int launch_repack(const uint8_t* src, uint8_t* dst, int type, int k, int n, uint64_t rb, int dir, hipStream_t s);
+int launch_repack(const uint8_t* src, uint8_t* dst, int type, int k, int n, int dir, hipStream_t s);
 int launch_dequant(const uint8_t* w, int type, int layout, int k, int n, uint64_t rb, const int32_t* rows, int nrows,
                    float* out, hipStream_t s);
 int launch_embed(const uint8_t* w, int type, int layout, int k, int n, uint64_t rb, const int32_t* tokens,

@@ -13,20 +13,123 @@
 namespace qk {
 namespace {
 
-// One work-group per (tile, super-block) group; threads stride over the group's bytes.
-// dir 0: GGUF -> T16 (gather), dir 1: T16 -> GGUF (scatter back).
-__global__ __launch_bounds__(256) void k_repack(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
-                                                int type, int nsb, uint64_t rb, int dir) {
-    const int bs = sb_bytes(type);
-    const int gbytes = 16 * bs;
-    const uint64_t tile = blockIdx.y, sb = blockIdx.x;
-    const uint64_t gofs = (tile * nsb + sb) * (uint64_t)gbytes;
-    for (int o = threadIdx.x; o < gbytes; o += blockDim.x) {
+// Repack: one work-group per (chunk of up to REPACK_SBS super-blocks, tile).  The chunk's 16 row windows
+// go through LDS in GGUF byte order, so that both sides of HBM see 16-byte accesses: GGUF rows as the
+// aligned words that cover them (a row of Q6_K blocks starts at any even byte; a tile's 16
+// rows, and so the tensor, end on a 16-byte boundary, so the words stay inside it), T16 groups as they
+// lie, one after another.  An LDS row keeps the window's offset in its word, so words move unshifted;
+// its stride is an odd number of words, so that the 16 rows a group's neighbouring pieces come from
+// fall into different banks.
+// Bound: HBM, each byte read and written once.  Measured (us, GGUF -> T16 / back; one byte per thread and
+// access before): Q4_K 5120 x 17408 60.8 -> 18.9 (5.3 TB/s) / 62.5 -> 21.5, Q6_K 17408 x 5120 103.5 -> 34.6 /
+// 119.8 -> 46.1, Q6_K 5120 x 248320 1460 -> 378 / 1636 -> 459.  Smaller chunks, down to one super-block where
+// the tiles are few, measured the same or slower (Q8_0 6144 x 5120 14.4 -> 15.6 at 1024 work-groups).
+constexpr int REPACK_SBS = 8;
+template <int TYPE>
+struct Repack {
+    static constexpr int BS = sb_bytes(TYPE), GB = group_bytes(TYPE), PIECES = GB / 16;
+    static constexpr int STRIDE = ((REPACK_SBS * BS + 15) / 16 + 1) / 2 * 32 + 16;  // bytes, an odd count of 16
+    // first byte past the planes whose 16-byte pieces are 16 bytes of one row (qs, ql, qh)
+    static constexpr int PLANES = TYPE == T_Q6_K ? 3072 : TYPE == T_Q8_0 ? 4096 : 2048;
+    // bytes that stay together outside the planes (d, dmin, scales)
+    static constexpr int UNIT = TYPE == T_Q6_K ? 1 : TYPE == T_Q8_0 ? 2 : 4;
+    static_assert(STRIDE >= REPACK_SBS * BS + (BS % 16 ? 16 : 0) && STRIDE / 16 % 2 == 1, "LDS row");
+    __device__ static bool plane(int o) { return o < PLANES || (TYPE == T_Q5_K && o >= 2304); }
+};
+
+// Bytes between LDS and registers at 2-byte alignment (16-byte where the type's blocks allow it).
+template <int TYPE>
+__device__ inline u4 lds_get16(const uint8_t* p) {
+    if constexpr (TYPE == T_Q4_K || TYPE == T_Q5_K) return *(const u4*)p;
+    u4 v;
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = *(const uint16_t*)(p + 4 * i) | ((uint32_t)*(const uint16_t*)(p + 4 * i + 2) << 16);
+    return v;
+}
+template <int TYPE>
+__device__ inline void lds_put16(uint8_t* p, const u4& v) {
+    if constexpr (TYPE == T_Q4_K || TYPE == T_Q5_K) {
+        *(u4*)p = v;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            *(uint16_t*)(p + 4 * i) = (uint16_t)v[i];
+            *(uint16_t*)(p + 4 * i + 2) = (uint16_t)(v[i] >> 16);
+        }
+    }
+}
+
+template <int TYPE, bool TO_T16>
+__global__ __launch_bounds__(256) void k_repack(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int nsb) {
+    using R = Repack<TYPE>;
+    using unit_t = std::conditional_t<R::UNIT == 4, uint32_t, std::conditional_t<R::UNIT == 2, uint16_t, uint8_t>>;
+    __shared__ __align__(16) uint8_t row[16 * R::STRIDE];
+    const uint64_t rb = (uint64_t)nsb * R::BS, tile = blockIdx.y;
+    const int s0 = (int)((uint64_t)blockIdx.x * nsb / gridDim.x), s1 = (int)((uint64_t)(blockIdx.x + 1) * nsb / gridDim.x);
+    const int len = (s1 - s0) * R::BS, words = (len + 15) / 16 + 1;  // a window covers at most that many
+    const uint64_t first = tile * 16 * rb + (uint64_t)s0 * R::BS;     // row r's window starts at first + r * rb
+    const uint64_t g0 = (tile * nsb + s0) * R::GB;                    // the chunk's groups in the T16 tensor
+    // byte o .. of group piece `i`: its place in the LDS rows
+    auto place = [&](int sb, int o) {
         int r, p;
-        t16_src(type, o, r, p);
-        const uint64_t gg = (tile * 16 + r) * rb + sb * bs + p;
-        if (dir == 0) dst[gofs + o] = src[gg];
-        else dst[gg] = src[gofs + o];
+        t16_src(TYPE, o, r, p);
+        return row + r * R::STRIDE + (int)((first + r * rb) & 15) + sb * R::BS + p;
+    };
+    if constexpr (TO_T16) {
+        // all of a thread's words are loaded before the first is stored; wave v takes rows v, v + 4, ...
+        constexpr int NW = R::STRIDE / 16, PASSES = (NW + 63) / 64;
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        u4 v[4][PASSES];
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int c = 0; c < PASSES; c++) {
+                const uint64_t a = first + (wave + 4 * q) * rb, at = (a & ~15ull) + 16 * (lane + 64 * c);
+                if (at < a + len) v[q][c] = ld16(src + at);
+            }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int c = 0; c < PASSES; c++) {
+                const uint64_t a = first + (wave + 4 * q) * rb, at = (a & ~15ull) + 16 * (lane + 64 * c);
+                if (at < a + len) *(u4*)(row + (wave + 4 * q) * R::STRIDE + 16 * (lane + 64 * c)) = v[q][c];
+            }
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < (s1 - s0) * R::PIECES; i += 256) {
+        const int sb = i / R::PIECES, o = 16 * (i - sb * R::PIECES);
+        u4 v;
+        if constexpr (!TO_T16) v = ld16(src + g0 + 16 * (uint64_t)i);
+        if (R::plane(o)) {
+            uint8_t* p = place(sb, o);
+            if constexpr (TO_T16) v = lds_get16<TYPE>(p);
+            else lds_put16<TYPE>(p, v);
+        } else {
+            unit_t u[16 / R::UNIT];
+            if constexpr (!TO_T16) __builtin_memcpy(u, &v, 16);
+#pragma unroll
+            for (int j = 0; j < 16 / R::UNIT; j++) {
+                unit_t* p = (unit_t*)place(sb, o + j * R::UNIT);
+                if constexpr (TO_T16) u[j] = *p;
+                else *p = u[j];
+            }
+            if constexpr (TO_T16) __builtin_memcpy(&v, u, 16);
+        }
+        if constexpr (TO_T16) *(u4*)(dst + g0 + 16 * (uint64_t)i) = v;
+    }
+    if constexpr (!TO_T16) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < 16 * words; i += 256) {
+            const int r = i / words, w = i - r * words;
+            const uint64_t a = first + r * rb, at = (a & ~15ull) + 16 * w;
+            const uint8_t* p = row + r * R::STRIDE + 16 * w;
+            if (at >= a && at + 16 <= a + len) {
+                *(u4*)(dst + at) = *(const u4*)p;
+            } else {  // the window's ends share their word with a neighbour's bytes
+                for (int j = 0; j < 16; j += 2)
+                    if (at + j >= a && at + j < a + len) *(uint16_t*)(dst + at + j) = *(const uint16_t*)(p + j);
+            }
+        }
     }
 }
 
@@ -249,9 +352,19 @@ __global__ __launch_bounds__(256) void k_synth(uint8_t* __restrict__ dst, int ty
 
 }  // namespace
 
-int launch_repack(const uint8_t* src, uint8_t* dst, int type, int k, int n, uint64_t rb, int dir, hipStream_t s) {
-    dim3 grid(k / 256, n / 16);
-    hipLaunchKernelGGL(k_repack, grid, dim3(256), 0, s, src, dst, type, k / 256, rb, dir);
+template <int TYPE>
+static void launch_repack_type(const uint8_t* src, uint8_t* dst, int nsb, int n, int dir, hipStream_t s) {
+    const dim3 grid((nsb + REPACK_SBS - 1) / REPACK_SBS, n / 16);
+    if (dir == 0) hipLaunchKernelGGL((k_repack<TYPE, true>), grid, dim3(256), 0, s, src, dst, nsb);
+    else hipLaunchKernelGGL((k_repack<TYPE, false>), grid, dim3(256), 0, s, src, dst, nsb);
+}
+
+int launch_repack(const uint8_t* src, uint8_t* dst, int type, int k, int n, int dir, hipStream_t s) {
+    if (type == T_Q4_K) launch_repack_type<T_Q4_K>(src, dst, k / 256, n, dir, s);
+    else if (type == T_Q5_K) launch_repack_type<T_Q5_K>(src, dst, k / 256, n, dir, s);
+    else if (type == T_Q6_K) launch_repack_type<T_Q6_K>(src, dst, k / 256, n, dir, s);
+    else if (type == T_Q8_0) launch_repack_type<T_Q8_0>(src, dst, k / 256, n, dir, s);
+    else return -1;
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
