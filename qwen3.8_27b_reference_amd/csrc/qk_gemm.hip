@@ -770,6 +770,23 @@ __global__ __launch_bounds__(THREADS) void k_gemm(const GemmMats mats, int nsb_r
     }
 }
 
+// Sum of part[j * stride], j < ks, in part order; U loads in flight at a time (past the last part: re-read,
+// not added).
+template <int U>
+__device__ inline f4 sum_parts(const f4* __restrict__ part, size_t stride, int ks) {
+    f4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j0 = 0; j0 < ks; j0 += U) {
+        f4 p[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) p[j] = part[min(j0 + j, ks - 1) * stride];
+        if (j0 == 0) v = p[0];
+#pragma unroll
+        for (int j = 0; j < U; j++)
+            if (j0 + j > 0 && j0 + j < ks) v += p[j];
+    }
+    return v;
+}
+
 // Adds the ks partial results [ks][m][n] of matrix blockIdx.y in part order (deterministic) into its y.
 struct SumMats {
     const f4* part[GEMM_MATS];
@@ -781,9 +798,7 @@ __global__ __launch_bounds__(256) void k_splitk_sum(const SumMats S, int ks) {
     f4* __restrict__ y = S.y[blockIdx.y];
     const size_t n4 = S.n4[blockIdx.y];
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
-        f4 v = part[i];
-        for (int j = 1; j < ks; j++) v += part[j * n4 + i];
-        y[i] = v;
+        y[i] = ks <= 4 ? sum_parts<4>(part + i, n4, ks) : sum_parts<8>(part + i, n4, ks);
     }
 }
 
@@ -793,11 +808,7 @@ __global__ __launch_bounds__(256) void k_splitk_sum(const SumMats S, int ks) {
 __global__ __launch_bounds__(256) void k_glu_sum(const f4* __restrict__ part, int ks, size_t n4, int n4row, void* y,
                                                  int yfmt) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
-        f4 g = part[i], u = part[(size_t)ks * n4 + i];
-        for (int j = 1; j < ks; j++) {
-            g += part[j * n4 + i];
-            u += part[(size_t)(ks + j) * n4 + i];
-        }
+        const f4 g = sum_parts<4>(part + i, n4, ks), u = sum_parts<4>(part + (size_t)ks * n4 + i, n4, ks);
         const int t = (int)(i / n4row), r = 4 * (int)(i % n4row);
         for (int e = 0; e < 4; e++) store_act(y, yfmt, (size_t)n4row * 4, t, r + e, g[e] / (1.0f + expf(-g[e])) * u[e]);
     }
