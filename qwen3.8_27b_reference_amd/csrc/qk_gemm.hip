@@ -28,55 +28,17 @@
 #include <atomic>
 
 #include "qk_device.h"
+#include "qk_dma.h"
 #include "qk_internal.h"
 
 namespace qk {
 namespace {
-
-#define LDS_AS __attribute__((address_space(3)))
 
 typedef float f16v __attribute__((ext_vector_type(16)));
 
 constexpr int THREADS = 512;  // 4 compute waves + 4 DMA waves (one of each per SIMD)
 constexpr int GEMM_MATS = 4;   // matrices of one grouped launch (the reference's gemv groups hold <= 4)
 constexpr int MAX_STAGES = 4;
-
-template <int N>
-__device__ inline void wait_vm() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-template <int N>
-__device__ inline void wait_vm_le(int n) {  // wait until at most n (<= N) operations are in flight
-    if constexpr (N > 0) {
-        if (n >= N) {
-            wait_vm<N>();
-            return;
-        }
-        wait_vm_le<N - 1>(n);
-    } else {
-        wait_vm<0>();
-    }
-}
-
-__device__ inline uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(LDS_AS const void*)p; }
-
-// 16 bytes per lane from global memory into LDS (M0 + 16 * lane), from inline assembly: the
-// compiler then holds no pending LDS-DMA, which it would wait out (vmcnt(0)) before LDS accesses it
-// cannot prove disjoint from the destination.  Every read of DMA'd bytes follows wait_vm* and a
-// barrier.  s_nop: M0 written by the SALU needs one wait state before an LDS-DMA reads it.
-__device__ inline void dma16(const void* g, uint8_t* lds) {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(lds_addr(lds)) : "memory");
-}
-
-// Work-group barrier that waits only for this wave's LDS operations: the release fence of
-// __syncthreads() would also wait for every LDS-DMA in flight, i.e. for the prefetched stages.
-__device__ inline void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
 
 // D(32x32 f32) += A(32x16 f16) * B(16x32 f16).  Lane l holds A[l & 31][8*(l >> 5) .. +7],
 // B[8*(l >> 5) .. +7][l & 31] and D[8*(v/4) + 4*(l >> 5) + v%4][l & 31] in register v (checked
@@ -195,16 +157,6 @@ struct Q4Src {
 
 __device__ inline Q4Src q4_src(const uint8_t* R) {  // R: the tile's piece 0 + 16 r + 8 h
     return Q4Src{ld8(R), ld8(R + 256)};
-}
-
-// Bytes 0,1 (lo) or 2,3 (hi) of v, each below 16, as an exact fp16 pair: read as FP8 E4M3 a byte
-// b < 16 is b * 2^-9 (subnormal for b < 8), so the scaled conversion by 2^9 gives b exactly
-// (checked for all 16 values on the device).  One instruction for the byte-perm + 1024 subtract.
-__device__ inline uint32_t nib_pair_lo(uint32_t v) {
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(v, 512.0f, false));
-}
-__device__ inline uint32_t nib_pair_hi(uint32_t v) {
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(v, 512.0f, true));
 }
 
 __device__ inline h8 q4_frag(const Q4Src& S4, uint32_t dm, int c) {  // dm: q4_dm of the chunk's sub-block
@@ -833,6 +785,27 @@ struct GemmCall {
     hipStream_t s;
 };
 
+// The second launch of a split call (ks parts) or a gate/up pair: adds the parts into the outputs.
+int launch_sums(const GemmCall& c, int ks) {
+    if (ks == 1 && !c.glu) return 0;
+    SumMats S{};
+    size_t off = 0, n4max = 0;
+    for (int z = 0; z < c.nz; z++) {
+        S.part[z] = (const f4*)(c.part + off);
+        S.y[z] = (f4*)c.y[z];
+        S.n4[z] = (size_t)c.m * c.n[z] / 4;  // n % 16 == 0
+        n4max = std::max(n4max, S.n4[z]);
+        off += (size_t)ks * c.m * c.n[z];
+    }
+    const int blocks = (int)std::min<size_t>((n4max + 255) / 256, 4096);
+    if (c.glu)
+        hipLaunchKernelGGL(k_glu_sum, dim3(blocks), dim3(256), 0, c.s, (const f4*)c.part, ks, S.n4[0], c.n[0] / 4, c.y[0],
+                           c.yfmt);
+    else
+        hipLaunchKernelGGL(k_splitk_sum, dim3(blocks, c.nz), dim3(256), 0, c.s, S, ks);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 template <int TYPE, int P, int NTB>
 int launch_p(const GemmCall& c, int ks) {
     constexpr size_t lds = GemmLds<TYPE, P, NTB>::TOTAL;
@@ -841,7 +814,6 @@ int launch_p(const GemmCall& c, int ks) {
     const int rep = XCDS / mblocks;
     const bool parts = ks > 1 || c.glu;
     GemmMats M{};
-    SumMats S{};
     int grid = 0;
     size_t off = 0;
     for (int z = 0; z < c.nz; z++) {
@@ -851,23 +823,12 @@ int launch_p(const GemmCall& c, int ks) {
         M.w[z] = c.w[z];
         M.n[z] = c.n[z];
         M.y[z] = parts ? c.part + off : (float*)c.y[z];
-        S.part[z] = (const f4*)(c.part + off);
-        S.y[z] = (f4*)c.y[z];
-        S.n4[z] = (size_t)c.m * c.n[z] / 4;  // n % 16 == 0
         off += (size_t)ks * c.m * c.n[z];
     }
     hipLaunchKernelGGL((k_gemm<TYPE, P, NTB>), dim3(grid, 1, c.nz), dim3(THREADS), lds, c.s, M, c.nsb,
                        c.xh, c.xperm, c.m, map, parts ? 1 : 0, ks);
     if (hipGetLastError() != hipSuccess) return -1;
-    size_t n4max = 0;
-    for (int z = 0; z < c.nz; z++) n4max = std::max(n4max, S.n4[z]);
-    const int blocks = (int)std::min<size_t>((n4max + 255) / 256, 4096);
-    if (c.glu)
-        hipLaunchKernelGGL(k_glu_sum, dim3(blocks), dim3(256), 0, c.s, (const f4*)c.part, ks, S.n4[0], c.n[0] / 4, c.y[0],
-                           c.yfmt);
-    else if (ks > 1)
-        hipLaunchKernelGGL(k_splitk_sum, dim3(blocks, c.nz), dim3(256), 0, c.s, S, ks);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    return launch_sums(c, ks);
 }
 
 // Plan: 32-token blocks per work-group NTB (1 up to 32 tokens, 2 up to 64, else 4), then the tile pairs
@@ -931,9 +892,48 @@ int launch_ntb(const GemmCall& c) {
     return -1;
 }
 
+// Up to 16 tokens: the weight-streaming form (qk_few.hip), where it has a plan and no knob asks for a plan
+// of this kernel.  Measured against this kernel at 5, 8, 13 and 16 tokens on 17 shapes: faster on every
+// one (us at 13 tokens: Q4_K 17408 x 5120 19.8 -> 16.8, Q6_K 27.1 -> 21.3, Q5_K 23.0 -> 20.0, Q8_0 6144 x 5120
+// 15.1 -> 12.4, the gate/up pair of 5120 x 17408 34.7 -> 26.6, the output projection 272 -> 214; least
+// gain Q4_K 1024 x 3072 x 2 7.9 -> 7.6).  Its x image has 16 token columns: above, this kernel's 32.
+// Returns 1 when it does not take the call.
+template <int TYPE>
+int launch_few_call(const GemmCall& c) {
+    if (g_gemm_p || g_gemm_ks) return 1;
+    FewParams p{};
+    size_t rows = 0;
+    for (int z = 0; z < c.nz; z++) {
+        p.w[z] = c.w[z];
+        p.n[z] = c.n[z];
+        p.tile0[z + 1] = p.tile0[z] + c.n[z] / 16;
+        rows += (size_t)c.n[z];
+    }
+    p.cnt = c.nz;
+    p.ntiles = p.tile0[c.nz];
+    p.nsb = c.nsb;
+    p.k = c.nsb * 256;
+    p.m = c.m;
+    p.x = c.xh;
+    p.xperm = c.xperm;
+    size_t lds = 0;
+    if (!few_plan(TYPE, p, c.cus, rows, c.part_cap, c.glu, lds)) return 1;
+    size_t off = 0;
+    for (int z = 0; z < c.nz; z++) {
+        p.y[z] = p.slices > 1 || c.glu ? c.part + off : (float*)c.y[z];
+        off += (size_t)p.slices * c.m * c.n[z];
+    }
+    if (launch_few(TYPE, p, lds, c.s) != 0) return -1;
+    return launch_sums(c, p.slices);
+}
+
 template <int TYPE>
 int launch_type(const GemmCall& c) {
     const int m = c.m;
+    if (m <= FEW_MAX_M) {
+        const int rc = launch_few_call<TYPE>(c);
+        if (rc <= 0) return rc;
+    }
     if (m <= 32) return launch_ntb<TYPE, 1>(c);
     if (m <= 64) return launch_ntb<TYPE, 2>(c);
     return launch_ntb<TYPE, 4>(c);

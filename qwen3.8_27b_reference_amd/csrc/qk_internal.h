@@ -117,6 +117,23 @@ int launch_gemm_group(int type, const uint8_t* const* ws, const int* ns, float* 
 // part (at least 2 m n floats), then k_glu_sum adds the parts and stores.  -1 when part is too small.
 int launch_gemm_glu(int type, const uint8_t* wg, const uint8_t* wu, int k, int n, const void* x, int xfmt, int m,
                     uint8_t* ximg, void* y, int yfmt, float* part, size_t part_cap, hipStream_t s);
+// Few-token GEMM (qk_few.hip, m <= FEW_MAX_M): all tiles of cnt matrices in one launch, `slices` K-slices x `wgs`
+// work-groups of `waves` waves.  y[z]: [slices][m][n[z]] fp32.
+constexpr int FEW_MAX_M = 16;
+struct FewParams {
+    const uint8_t* w[GEMV_MAX_CNT];
+    float* y[GEMV_MAX_CNT];
+    int n[GEMV_MAX_CNT];
+    int tile0[GEMV_MAX_CNT + 1];
+    int cnt, ntiles, nsb, k, m;
+    const _Float16* x;
+    int xperm;
+    int slices, wgs, waves, lds_ring;
+};
+// Fills slices, wgs, waves, lds_ring and the LDS size; false when no plan fits (rows: of all matrices;
+// part_cap: floats for [slices][m][rows]; sums: the slices are added by a second launch even if one).
+bool few_plan(int type, FewParams& p, int cus, size_t rows, size_t part_cap, bool sums, size_t& lds);
+int launch_few(int type, const FewParams& p, size_t lds, hipStream_t s);
 void gemm_set_map(int map);  // tuning: 1 = one token block per XCD (default), 0 = a unit's token blocks on one XCD
 bool gemm_set_pairs(int p);  // tuning override of the tile pairs per work-group (0 = planned)
 bool gemm_set_ksplit(int ks);  // tuning override of the K-parts (0 = planned, 1..16)
