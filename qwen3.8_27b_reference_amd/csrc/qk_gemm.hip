@@ -66,12 +66,11 @@ __global__ __launch_bounds__(256) void k_gemm_cvt_x(const float* __restrict__ x,
     }
 }
 
-// Byte offset of lane l's B operand (chunk 0) inside a 32-token block's 4 KiB of one stage.
-__device__ inline int xb_lane_off(int lane) {
-    const int t = lane & 31, h = lane >> 5, j = t >> 3;
-    return 1024 * j + 128 * (h ^ (j & 1)) + 16 * (t & 7);
+// Byte offset of lane l's B operand of chunk c inside a 32-token block's 4 KiB of one stage.
+__device__ inline int xb_lane_off(int lane, int c) {
+    const int t = lane & 31, h = lane >> 5;
+    return 128 * t + ((16 * (h ^ ((t >> 1) & 7))) ^ (32 * c));
 }
-
 
 // ------------------------------------------------------------------------------------------------
 // Raw bytes of one step (quarter q of super-block sb) of one tile, staged in LDS by LDS-DMA as
@@ -513,7 +512,7 @@ __global__ __launch_bounds__(THREADS) void k_gemm(const GemmMats mats, int nsb_r
                     for (int j = 0; j < SHP; j++) sp[j] = gemm_src<TYPE>(sR(st) + tile(j) * L::RPIECES * 256, q, r, h);
 #pragma unroll
                     for (int c = 0; c < 4; c++)
-                        bx[c] = __builtin_bit_cast(h8, *(const u4*)(sX(st) + wave * 4096 + xb_lane_off(lane) + 256 * c));
+                        bx[c] = __builtin_bit_cast(h8, *(const u4*)(sX(st) + wave * 4096 + xb_lane_off(lane, c)));
                 }
             }
             if (s + STAGES - 1 < steps) issue_step(s + STAGES - 1);
@@ -568,11 +567,11 @@ __global__ __launch_bounds__(THREADS) void k_gemm(const GemmMats mats, int nsb_r
     // 8 (p >> 2)) and each step adds a part uniform over the wave.
     const uint8_t* xb[XPW];
     {
-        const int p = 2 * (lane >> 4) + (((lane >> 3) & 1) ^ (wave & 1));
+        const int p = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
         const int pe = xperm ? 256 * (p & 3) + 8 * (p >> 2) : 256 * sb0 + 8 * p;
 #pragma unroll
         for (int tb = 0; tb < XPW; tb++) {
-            const int tok = min(32 * (tb0 + tb) + 8 * wave + (lane & 7), m - 1);
+            const int tok = min(32 * (tb0 + tb) + 8 * wave + (lane >> 3), m - 1);
             xb[tb] = (const uint8_t*)(xh + (size_t)tok * kx + pe);
         }
     }
@@ -597,7 +596,7 @@ __global__ __launch_bounds__(THREADS) void k_gemm(const GemmMats mats, int nsb_r
     h8 a[2][NPL], b[OWN > 0 ? NTB : 1], bs;
     auto tile_idx = [&](int i) { return 2 * pair_of(i) + u; };
     // per-lane LDS bases: every step adds its stage offset once, the rest are immediate offsets
-    const uint8_t* const xlane = smem + xb_lane_off(lane);
+    const int xl = xb_lane_off(lane, 0);
     const uint8_t* const rown = sR(0) + (2 * wave * OWN + u) * L::RPIECES * 256 + 16 * r + 8 * h;
     const uint8_t* const rsh = sR(0) + (8 * OWN + u) * L::RPIECES * 256 + 16 * r + 8 * h;
     auto load_src = [&](int t) {
@@ -622,7 +621,7 @@ __global__ __launch_bounds__(THREADS) void k_gemm(const GemmMats mats, int nsb_r
         }
     };
     auto load_x = [&](int t, int c, int tb) {  // B operand: token block tb, chunk c of step t
-        return __builtin_bit_cast(h8, *(const u4*)(xlane + (t % STAGES) * L::STAGE + tb * 4096 + 256 * c));
+        return __builtin_bit_cast(h8, *(const u4*)(smem + ((xl + (t % STAGES) * L::STAGE) ^ (32 * c)) + tb * 4096));
     };
     auto frag = [&](int i, int q, int c) {
         return gemm_frag<TYPE>(src[i], sc4[GT<TYPE>::SP > 0 ? i : 0], C::DM ? dmc[i] : 0u, q, c);
