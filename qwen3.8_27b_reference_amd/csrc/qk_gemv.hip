@@ -1370,7 +1370,7 @@ int dispatch(int type, int na, int m, F&& f) {
 std::atomic<int> g_tune_waves{0};
 std::atomic<bool> g_fused{true};  // m <= 4 through the int8 kernel where its plan applies
 std::atomic<int> g_wpg{0};        // at most this many waves per int8 work-group (0 = as many as fit)
-std::atomic<int> g_img_kib{32};   // largest activation image per range before the K-slices double
+std::atomic<int> g_img_kib{0};    // largest activation image per range before the K-slices double (0 = planned)
 std::atomic<int> g_dshift{1};     // int8 kernel: about nu >> g_dshift of a range's units handed out dynamically
 std::atomic<int> g_min_waves{0};  // int8 kernel at m >= 2: the fewest waves per work-group it is planned with
 std::atomic<int> g_max_slots{8};  // int8 kernel: the most token slots per launch (4 or 8)
@@ -1436,7 +1436,9 @@ struct Fused {
         // fit the LDS, or leave it room for fewer than WANT waves: a range's unit sums and table grow
         // with its units (a 248320-row matrix left four waves per CU at one work-group per CU, and
         // nine at two, in two rounds)
-        constexpr int WANT = 8;
+        // A pair of one or two tokens stays in one round down to four waves (a wave's ring is twice as
+        // large: Q6_K 5120 x 17408 at one token took four rounds of seven waves, 38.7 us against 29.2).
+        constexpr int WANT = NA == 2 && MT <= 2 ? 4 : 8;
         GemvParams best = p;
         int best_w = 0;
         size_t best_lds = 0;
@@ -1444,7 +1446,7 @@ struct Fused {
             GemvParams t = p;
             int w = 0;
             size_t l = 0;
-            if (plan_groups(t, groups, MT == 8 ? 32 : 16, w, l) && w > best_w) {
+            if (plan_groups(t, groups, groups <= cus, MT == 8 ? 32 : 16, w, l) && w > best_w) {
                 best = t;
                 best_w = w;
                 best_lds = l;
@@ -1485,16 +1487,36 @@ struct Fused {
         for (int ci = 0; ci < nc; ci++) {
             const Cand& c = cands[ci];
             GemvParams t = p;
-            if (plan_groups(t, c.g, c.S, wpg, lds, c.S)) {
+            if (plan_groups(t, c.g, true, c.S, wpg, lds, c.S)) {
                 p = t;
                 return true;
             }
         }
         return false;
     }
-    // Plan for `groups` work-groups: the fewest slices (from smin, at most smax) whose range image
-    // fits 32 KB, else the smallest image.
-    static bool plan_groups(GemvParams& p, int groups, int smax, int& wpg, size_t& lds, int smin = 1) {
+    // Waves per work-group where the LDS holds w, for ranges of nu units that convert `jobs` (token, super-
+    // block) pairs.  As many as fit is not the fastest: a work-group's waves start ~85 ns apart and a
+    // SIMD with one wave more than the others ends last, so a multiple of four below the most is taken
+    // (us at one token: Q4_K 5120 x 17408 16 waves 12.64, 14 12.8, 12 11.70, 10 12.18, 8 12.46; Q6_K 13 waves
+    // 16.19, 12 15.33, 8 15.36; Q8_0 8192 x 4096 10 waves 9.00, 8 8.71; at four tokens Q4_K 5120 x 5120 16
+    // waves 9.25, 12 8.81), and eight for a range of a few units (Q4_K 1024 x 3072, three units: 16 waves
+    // 6.13, 12 5.55, 8 5.01).  Kept at the most: ranges with more conversions than three a wave (Q4_K
+    // 11008 x 4096, 43: 16 waves 8.93, 12 9.12), many thin slices (Q8_0 11008 x 4096 at two tokens, 43 slices: 11 waves 21.4, 8 24.0), several rounds of
+    // work-groups (Q6_K 5120 x 100000 at two
+    // tokens 11 waves 81.3, 8 84.0) and pairs of two tokens and more, whose unit math is the bound (Q4_K
+    // 5120 x 17408 at four 11 waves 24.9, 8 27.1).
+    static int pick_waves(int w, int S, int nu, int jobs, bool one_round) {
+        if (MT == 8 || (NA == 2 && MT > 1)) return w;
+        if (jobs <= 36 && S <= 8 && one_round) {
+            if (nu < 16) return std::min(w, 8);
+            return w >= 12 ? 12 : w >= 8 ? 8 : w;
+        }
+        return w > 12 && w < 16 ? 12 : w;
+    }
+    // Plan for `groups` work-groups: the fewest slices (from smin, at most smax) whose range image fits
+    // 20 KB at one token (Q4_K 17408 x 5120: four slices 12.3 us, two 13.2), 32 KB at two and four (Q8_0
+    // 5120 x 17408 at two: one slice 19.0, two 19.8), else the smallest image.
+    static bool plan_groups(GemvParams& p, int groups, bool one_round, int smax, int& wpg, size_t& lds, int smin = 1) {
         const int ntiles = p.units / p.nsb;
         int best = 0;
         size_t best_img = 0;
@@ -1510,16 +1532,27 @@ struct Fused {
             }
             // eight token slots: an image twice the size (the slices' exchange levels cost more than
             // the waves the larger image takes)
-            if (img <= (size_t)g_img_kib.load() * 1024 * (MT == 8 ? 2 : 1)) break;
+            const int kib = g_img_kib.load() > 0 ? g_img_kib.load() : MT == 1 ? 20 : 32;
+            if (img <= (size_t)kib * 1024 * (MT == 8 ? 2 : 1)) break;
         }
         if (!best) return false;
         for (int waves = std::min(g_wpg.load() > 0 ? g_wpg.load() : 16, gemv1_max_waves<MT>()); waves >= 4; waves--) {
             GemvParams t = p;
             const size_t total = layout(t, groups, best, waves);
             if (total && total <= (size_t)LDS_PER_CU) {
-                p = t;
                 wpg = waves;
                 lds = total;
+                if (g_wpg.load() == 0) {
+                    const int w = pick_waves(waves, best, (p.units + groups - 1) / groups, t.lds_part / G1<TYPE, MT>::IMG * MT,
+                                             one_round);
+                    GemvParams f = p;
+                    if (const size_t fewer = w < waves ? layout(f, groups, best, w) : 0) {
+                        t = f;
+                        wpg = w;
+                        lds = fewer;
+                    }
+                }
+                p = t;
                 return true;
             }
         }
@@ -1563,7 +1596,7 @@ struct Fused {
 void gemv_set_waves(int waves) { g_tune_waves = waves; }
 void gemv_set_fused(bool on) { g_fused = on; }
 void gemv_set_wpg(int w) { g_wpg = w; }
-void gemv_set_img_kib(int kib) { g_img_kib = kib > 0 ? kib : 32; }
+void gemv_set_img_kib(int kib) { g_img_kib = kib; }
 void gemv_set_dshift(int sh) { g_dshift = sh; }
 void gemv_set_min_waves(int w) { g_min_waves = w; }
 void gemv_set_max_slots(int t) { g_max_slots = t; }
