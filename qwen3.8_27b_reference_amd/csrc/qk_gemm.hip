@@ -367,6 +367,7 @@ struct GemmMats {
     const uint8_t* w[GEMM_MATS];
     float* y[GEMM_MATS];
     int n[GEMM_MATS];
+    int ldy;  // floats between consecutive tokens of y[0] (a call's part of a matrix); 0: n[z]
 };
 
 template <int TYPE, int P, int NTB>
@@ -407,6 +408,7 @@ __global__ __launch_bounds__(THREADS) void k_gemm(const GemmMats mats, int nsb_r
     const int kx = nsb_row * 256;  // K: halves between consecutive tokens of x
     const int steps = nsb * 4;
     float* const y = mats.y[z] + (parts ? (size_t)part * m * n : 0);
+    const int ldy = mats.ldy ? mats.ldy : n;
 
     // DMA jobs of step t.  Activations: XJ jobs (token block tb, tokens 8j .. 8j + 7), compute wave w
     // issuing job j = w of every token block, just before its barrier where it would wait anyway.  Weights:
@@ -427,7 +429,7 @@ __global__ __launch_bounds__(THREADS) void k_gemm(const GemmMats mats, int nsb_r
         for (int j = 0; j < 4; j++) {
             const int row = 8 * j + 4 * h;  // within the pair
             if (2 * pair + (row >> 4) < tn)
-                *(f4*)(y + (size_t)tok * n + (size_t)tile0 * 16 + 32 * pair + row) =
+                *(f4*)(y + (size_t)tok * ldy + (size_t)tile0 * 16 + 32 * pair + row) =
                     f4{v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]};
         }
     };
@@ -743,13 +745,15 @@ struct SumMats {
     const f4* part[GEMM_MATS];
     f4* y[GEMM_MATS];
     size_t n4[GEMM_MATS];
+    int n4row, ldy4;  // a part of a matrix (ldy4 != 0): f4s of its rows, and between tokens of y[0]
 };
 __global__ __launch_bounds__(256) void k_splitk_sum(const SumMats S, int ks) {
     const f4* __restrict__ part = S.part[blockIdx.y];
     f4* __restrict__ y = S.y[blockIdx.y];
     const size_t n4 = S.n4[blockIdx.y];
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
-        y[i] = ks <= 4 ? sum_parts<4>(part + i, n4, ks) : sum_parts<8>(part + i, n4, ks);
+        const size_t o = S.ldy4 ? i / S.n4row * S.ldy4 + i % S.n4row : i;
+        y[o] = ks <= 4 ? sum_parts<4>(part + i, n4, ks) : sum_parts<8>(part + i, n4, ks);
     }
 }
 
@@ -782,6 +786,7 @@ struct GemmCall {
     size_t part_cap;
     int cus;
     hipStream_t s;
+    int ldy;  // floats between consecutive tokens of y[0] where the call is part of a matrix; 0: n
 };
 
 // The second launch of a split call (ks parts) or a gate/up pair: adds the parts into the outputs.
@@ -796,6 +801,8 @@ int launch_sums(const GemmCall& c, int ks) {
         n4max = std::max(n4max, S.n4[z]);
         off += (size_t)ks * c.m * c.n[z];
     }
+    S.n4row = c.n[0] / 4;
+    S.ldy4 = c.ldy / 4;
     const int blocks = (int)std::min<size_t>((n4max + 255) / 256, 4096);
     if (c.glu)
         hipLaunchKernelGGL(k_glu_sum, dim3(blocks), dim3(256), 0, c.s, (const f4*)c.part, ks, S.n4[0], c.n[0] / 4, c.y[0],
@@ -824,6 +831,7 @@ int launch_p(const GemmCall& c, int ks) {
         M.y[z] = parts ? c.part + off : (float*)c.y[z];
         off += (size_t)ks * c.m * c.n[z];
     }
+    M.ldy = parts ? 0 : c.ldy;
     hipLaunchKernelGGL((k_gemm<TYPE, P, NTB>), dim3(grid, 1, c.nz), dim3(THREADS), lds, c.s, M, c.nsb,
                        c.xh, c.xperm, c.m, map, parts ? 1 : 0, ks);
     if (hipGetLastError() != hipSuccess) return -1;
@@ -851,15 +859,25 @@ constexpr int MAX_KS = 16;
 std::atomic<int> g_gemm_p{0};   // tuning override of the tile pairs per work-group (0 = planned)
 std::atomic<int> g_gemm_ks{0};  // tuning override of the K-parts (0 = planned)
 
+struct GemmPlan {
+    int p = 0, ks = 0;
+    double t = 0.0;  // estimated us
+};
+
 template <int TYPE, int NTB>
-int launch_ntb(const GemmCall& c) {
-    const int nsb = c.nsb, m = c.m, cus = c.cus;
+double step_us(int p, int sbs) {  // a work-group's steps over sbs super-blocks
     const double wkib = (GT<TYPE>::RP * 512.0 + GT<TYPE>::SP * 128.0) / 1024.0;  // per pair and step
+    const double t = sbs * 4 * (4.0 * NTB + p * wkib) * 0.03;
+    return p % 4 == 1 ? t * 1.3 : t;  // P = 5, 9: the DMA waves also multiply a pair
+}
+
+template <int TYPE, int NTB>
+GemmPlan plan_ntb(const GemmCall& c) {
+    const int nsb = c.nsb, m = c.m, cus = c.cus;
     const int mblocks = (m + 32 * NTB - 1) / (32 * NTB);
     size_t nsum = 0;  // rows of all the matrices
     for (int z = 0; z < c.nz; z++) nsum += (size_t)c.n[z];
-    int best_p = 0, best_ks = 0;
-    double best_t = 0.0;
+    GemmPlan best;
     for (int p : P_CHOICES) {
         if (g_gemm_p ? p != g_gemm_p : NTB < 4 && p != 4 && p != 8) continue;
         for (int ks = 1; ks <= MAX_KS && ks <= nsb; ks++) {
@@ -868,27 +886,62 @@ int launch_ntb(const GemmCall& c) {
             long long wgs = 0;
             for (int z = 0; z < c.nz; z++) wgs += (long long)(((c.n[z] / 16 + 1) / 2 + p - 1) / p) * mblocks * ks;
             const long long busy = (wgs + cus - 1) / cus;
-            const int sbw = (nsb + ks - 1) / ks;
-            double step = sbw * 4 * (4.0 * NTB + p * wkib) * 0.03;
-            if (p % 4 == 1) step *= 1.3;  // P = 5, 9: the DMA waves also multiply a pair
-            const double t = busy * (step + 5.0) +
+            const double t = busy * (step_us<TYPE, NTB>(p, (nsb + ks - 1) / ks) + 5.0) +
                              (ks > 1 || c.glu ? (ks + 1) * 4.0 * m * (double)nsum / 5e6 + 2.0 : 0.0);
-            if (!best_p || t < best_t) {
-                best_p = p;
-                best_ks = ks;
-                best_t = t;
+            if (!best.p || t < best.t) best = {p, ks, t};
+        }
+    }
+    return best;
+}
+
+template <int TYPE, int NTB>
+int launch_plan(const GemmCall& c, const GemmPlan& pl) {
+    switch (pl.p) {
+        case 2: return launch_p<TYPE, 2, NTB>(c, pl.ks);
+        case 3: return launch_p<TYPE, 3, NTB>(c, pl.ks);
+        case 4: return launch_p<TYPE, 4, NTB>(c, pl.ks);
+        case 5: return launch_p<TYPE, 5, NTB>(c, pl.ks);
+        case 8: return launch_p<TYPE, 8, NTB>(c, pl.ks);
+        case 9: return launch_p<TYPE, 9, NTB>(c, pl.ks);
+    }
+    return -1;
+}
+
+template <int TYPE, int NTB>
+int launch_ntb(const GemmCall& c) {
+    const GemmPlan one = plan_ntb<TYPE, NTB>(c);
+    if constexpr (NTB == 4) {
+        // A call of more than one round of work-groups ends in a round that only part of the CUs share:
+        // where it is estimated faster, its whole rounds run as one launch (P = 8) and the rows left over as
+        // a second with a plan of their own, whose K-parts fill the CUs.  The estimate here is the plan's with
+        // what single calls hide in the ranking: P = 8 rounds at 1.13 of it (72..74 us for 65 at K = 5120), 8 us
+        // for the second launch and its sum, partials written and read; and 5 % in its favour.  Measured (us,
+        // one launch / two): Q8_0 6144 x 5120 at 2048 tokens 174 / 138, Q4_K 17408 x 5120 389 / 340, Q6_K
+        // 17408 x 5120 486 / 437, Q4_K 5120 x 17408 at 640 134 / 121, at 2048 363 / 347; below the line Q4_K 5120 x
+        // 17408 at 1024 181 / 186 and at 1500 265 / 277, which stay single.
+        constexpr int P = 8;
+        const int mblocks = (c.m + 32 * NTB - 1) / (32 * NTB), px = ((c.n[0] / 16 + 1) / 2 + P - 1) / P;
+        // whole rounds on every XCD: both maps give it px0 / 8 (or px0 mblocks / 8) whole units
+        const int rounds = (int)((long long)px * mblocks / c.cus), px0 = c.cus / XCDS * rounds / mblocks * XCDS;
+        if (c.nz == 1 && !c.glu && !g_gemm_p && !g_gemm_ks && rounds >= 1 && px0 >= 1 && px0 < px) {
+            const int rows = px0 * P * 32;
+            GemmCall a = c, b = c;
+            a.n[0] = rows;
+            b.n[0] = c.n[0] - rows;
+            b.w[0] = c.w[0] + (size_t)(rows / 16) * c.nsb * Gcfg<TYPE>::GBYTES;
+            b.y[0] = (float*)c.y[0] + rows;
+            a.ldy = b.ldy = c.n[0];
+            const GemmPlan tail = plan_ntb<TYPE, NTB>(b);
+            auto us = [](const GemmPlan& pl) { return pl.p % 4 == 1 ? pl.t : 1.13 * pl.t; };
+            const double two = 1.13 * rounds * (step_us<TYPE, NTB>(P, c.nsb) + 5.0) + us(tail) + 8.0 +
+                               (tail.ks > 1 ? tail.ks * 4.0 * c.m * (double)b.n[0] / 5e6 : 0.0);
+            if (1.05 * two < us(one)) {
+                const int rc = launch_p<TYPE, P, NTB>(a, 1);
+                return rc != 0 ? rc : launch_plan<TYPE, NTB>(b, tail);
             }
         }
     }
-    switch (best_p) {
-        case 2: return launch_p<TYPE, 2, NTB>(c, best_ks);
-        case 3: return launch_p<TYPE, 3, NTB>(c, best_ks);
-        case 4: return launch_p<TYPE, 4, NTB>(c, best_ks);
-        case 5: return launch_p<TYPE, 5, NTB>(c, best_ks);
-        case 8: return launch_p<TYPE, 8, NTB>(c, best_ks);
-        case 9: return launch_p<TYPE, 9, NTB>(c, best_ks);
-    }
-    return -1;
+    return launch_plan<TYPE, NTB>(c, one);
 }
 
 // Up to 16 tokens: the weight-streaming form (qk_few.hip), where it has a plan and no knob asks for a plan
