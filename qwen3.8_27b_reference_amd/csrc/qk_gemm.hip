@@ -966,7 +966,7 @@ int launch_few_call(const GemmCall& c) {
     p.nsb = c.nsb;
     p.k = c.nsb * 256;
     p.m = c.m;
-    p.x = c.xh;
+    p.x = (const uint16_t*)c.xh;
     p.xperm = c.xperm;
     size_t lds = 0;
     if (!few_plan(TYPE, p, c.cus, rows, c.part_cap, c.glu, lds)) return 1;

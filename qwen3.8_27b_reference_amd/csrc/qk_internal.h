@@ -126,7 +126,7 @@ struct FewParams {
     int n[GEMV_MAX_CNT];
     int tile0[GEMV_MAX_CNT + 1];
     int cnt, ntiles, nsb, k, m;
-    const _Float16* x;
+    const uint16_t* x;  // fp16
     int xperm;
     int slices, wgs, waves, lds_ring;
 };
