@@ -10,7 +10,7 @@
 //  * k_f32_rows: one work-group per 1, 2 or 4 rows, k split over its 256 threads, up to 16 tokens per
 //    pass.  n = 48, k = 5120 (us per call, graph-timed, one wave per row before): one token 10.4 ->
 //    2.6 (~2 of them the launch), 13 tokens 66 -> 3.3, 512 tokens 3540 -> 12.3.
-//  * k_f32_tile: fp32 MFMA on tiles of 32 rows x 32 tokens, k split over the sixteen waves of the
+//  * k_f32_tile: fp32 MFMA on tiles of 16 x 16 or 32 x 32 (rows x tokens), k split over the sixteen waves of the
 //    work-group, their sums added through LDS in wave order.  n = 1024, m = 512 58 us (93 TFLOP/s);
 //    bounded by the operand loads (a lane's 16 bytes are a line of their own) as much as by the MFMAs.
 #include <algorithm>
@@ -182,6 +182,12 @@ void launch_fmt(const F32Mats& M, int cnt, int k, const void* x, int m, hipStrea
     //    m = 2048, 30.1 against 20.1 at m = 1000; n = 1024: 31.0 against 37.7 at m = 128), with more
     //    than the 16 tokens that one pass of the row kernel takes (n = 17408: 115.7 against 100.0 at
     //    m = 16, 118.8 against 183.8 at m = 20).
+    //  * Tiles of 16 x 16 pay from 44 Ki outputs while they run in one round over the CUs (256 tiles): a
+    //    work-group's time is its own 32 lines of k, whatever the call (us, rows / tiles on fp16 x: n = 48, m =
+    //    1000 21.0 / 16.3, n = 128, m = 512 24.5 / 16.4, n = 1024, m = 64 24.1 / 16.3, n = 4096, m = 13 29.8 /
+    //    23.1, at k = 1024 11.9 / 6.7; on fp32 x 29.3 / 20.4 for the first; below the line n = 48, m = 760 23.3 /
+    //    20.4 but n = 128, m = 300 18.2 / 20.4; two rounds, n = 48, m = 1500: 29.6 / 31.2).  One rule for
+    //    every format, so that they give the same bits.
     //  * Weights beyond the L2s (32 MiB) are read once: 16 tokens a pass (n = 17408, m = 16: 100.0
     //    against 138.1 with eight, 232.0 with four).
     //  * Four tokens a pass spread a small call over the most work-groups; eight pay once 8192 passes are
@@ -191,6 +197,9 @@ void launch_fmt(const F32Mats& M, int cnt, int k, const void* x, int m, hipStrea
     //    row 3.29, two 3.78; m = 64 4.50 / 4.41 / four 4.61; m = 256 10.8 / 7.9 / 7.25).
     // (Past 2^23 rows a work-group per row would exceed a grid's 2^32 threads.)
     if ((m > 16 && rows * m >= 96 * 1024) || nmax > (1 << 23)) return launch_tile<FMT, 2>(M, nmax, cnt, k, x, m, s);
+    long long tiles = 0;
+    for (int z = 0; z < cnt; z++) tiles += (long long)((M.n[z] + 15) / 16) * ((m + 15) / 16);
+    if (rows * m >= 44 * 1024 && tiles <= 256) return launch_tile<FMT, 1>(M, nmax, cnt, k, x, m, s);
     if (m == 1) return launch_rows<FMT, 1, 1>(M, nmax, cnt, k, x, m, s);
     if (m > 8 && m <= 16 && rows * k > (8ll << 20)) return launch_rows<FMT, 4, 16>(M, nmax, cnt, k, x, m, s);
     const long long passes = rows * ((m + 3) / 4);

@@ -32,7 +32,9 @@ def _weights(n, k, seed):
 # (k, n, m): rows 1 / 2 / 4 per work-group, four, eight and sixteen tokens a pass, MFMA tiles
 SHAPES = [(256, 1, 1), (1280, 3, 2), (5120, 48, 4), (768, 5, 5), (256, 17, 9), (5120, 48, 13), (1024, 130, 17),
           (1280, 127, 22), (256, 1031, 8), (1024, 2050, 15), (256, 4099, 6), (8448, 1030, 13), (256, 97, 1025),
-          (1280, 1601, 63), (768, 33, 3001)]
+          (1280, 1601, 63), (768, 33, 3001),
+          # 16 x 16 tiles: at 256 tiles and one past, ragged rows and tokens, on the line of 44 Ki outputs
+          (1280, 4096, 11), (256, 4091, 16), (768, 4097, 13), (2304, 44, 1024), (256, 47, 1013), (5120, 241, 255)]
 
 
 @pytest.mark.parametrize("k,n,m", SHAPES, ids=[f"k{k}n{n}m{m}" for k, n, m in SHAPES])
