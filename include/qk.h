@@ -211,9 +211,10 @@ int qk_gemv_plan(const qk_weight* const* ws, int32_t cnt, int32_t glu, int32_t m
  * whose domain is |x| < 65504 with Q4_K 32-element sub-block sums below that too, for comparisons
  * only; Q8_0 / Q5_K always take the int8 kernel),
  * "gemv_wpg" (at most this many waves, 4..16, per int8-kernel work-group; 0 = as many as the LDS
- * holds), "gemv_img_kib" (int8 kernel: the K-slices double until a range's activation image fits this
- * many KiB, 1..160; 0 restores the plan's own: 20 at one token, 32 above), "gemv_dshift" (int8 kernel: about nu >> value of a work-group's nu
- * units are handed out by a counter, the rest statically; 0..31, default 1), "gemv_min_waves" (int8
+ * holds), "gemv_img_kib" (int8 kernel: the fewest K-slices whose activation image per range fits this
+ * many KiB, 1..160; 0 restores the plan's own 32 and its choice of more slices at one token), "gemv_dshift"
+ * (int8 kernel: about nu >> value of a work-group's nu units are handed out by a counter, the rest
+ * statically; 0..31, default 1), "gemv_min_waves" (int8
  * kernel at m >= 2: the fewest waves per work-group its plan may leave before Q4_K / Q6_K calls go to
  * the general kernel; 0..16, default 0), "gemv_token_slots" (int8 kernel: the most tokens one launch
  * carries, 8 (default: one weight pass per eight tokens) or 4 (m = 5..8 as four tokens and the rest)),

@@ -1370,7 +1370,7 @@ int dispatch(int type, int na, int m, F&& f) {
 std::atomic<int> g_tune_waves{0};
 std::atomic<bool> g_fused{true};  // m <= 4 through the int8 kernel where its plan applies
 std::atomic<int> g_wpg{0};        // at most this many waves per int8 work-group (0 = as many as fit)
-std::atomic<int> g_img_kib{0};    // largest activation image per range before the K-slices double (0 = planned)
+std::atomic<int> g_img_kib{0};    // a range's largest activation image before more K-slices (0 = the plan's bound)
 std::atomic<int> g_dshift{1};     // int8 kernel: about nu >> g_dshift of a range's units handed out dynamically
 std::atomic<int> g_min_waves{0};  // int8 kernel at m >= 2: the fewest waves per work-group it is planned with
 std::atomic<int> g_max_slots{8};  // int8 kernel: the most token slots per launch (4 or 8)
@@ -1429,8 +1429,6 @@ struct Fused {
         p.lds_ring = (int)align16(p.lds_tab + 16 * (size_t)maxnu);
         return p.lds_ring + (size_t)waves * D * NA * C::GB;
     }
-    // Slices: the fewest whose range image fits 32 KB (else the smallest image), then as many waves
-    // (<= 16) as the LDS left feeds.
     static bool plan(GemvParams& p, int cus, bool small, int& wpg, size_t& lds) {
         // one work-group per CU; more (smaller ranges, run in rounds) when one range's tables do not
         // fit the LDS, or leave it room for fewer than WANT waves: a range's unit sums and table grow
@@ -1513,27 +1511,43 @@ struct Fused {
         }
         return w > 12 && w < 16 ? 12 : w;
     }
-    // Plan for `groups` work-groups: the fewest slices (from smin, at most smax) whose range image fits
-    // 20 KB at one token (Q4_K 17408 x 5120: four slices 12.3 us, two 13.2), 32 KB at two and four (Q8_0
-    // 5120 x 17408 at two: one slice 19.0, two 19.8), else the smallest image.
+    // Plan for `groups` work-groups: the fewest slices (from smin, at most smax) whose range image fits 32 KB
+    // (64 with eight token slots: the slices' exchange levels cost more than the waves the larger image
+    // takes), else the smallest image.  The count divides the super-blocks, so a lower bound would jump to many
+    // slices where they have few divisors (one token, 20 KB against 32, us: Q4_K 6656 x 11888 13 slices 16.1, one
+    // 11.4; 9984 x 5120 13 slices 12.7, three 10.0; 6400 x 17408 five slices 16.7, one 13.9; Q5_K, Q6_K and Q8_0
+    // alike); the knob gemv_img_kib sets another.
     static bool plan_groups(GemvParams& p, int groups, bool one_round, int smax, int& wpg, size_t& lds, int smin = 1) {
         const int ntiles = p.units / p.nsb;
-        int best = 0;
-        size_t best_img = 0;
-        for (int S = smin; S <= smax && S <= p.nsb; S++) {
+        auto image = [&](int S) -> size_t {  // of the largest range; 0 when S slices are not possible
             GemvParams t = p;
             if (p.nsb % S || (size_t)ntiles * xnodes_of(S) * MT * 16 > p.xslot_cap ||
                 !layout(t, groups, S, gemv1_max_waves<MT>()))
-                continue;
-            const size_t img = (size_t)t.lds_part;
-            if (!best || img < best_img) {
+                return 0;
+            return (size_t)t.lds_part;
+        };
+        const int knob = g_img_kib.load();
+        const size_t bound = (size_t)(knob > 0 ? knob : 32) * 1024 * (MT == 8 ? 2 : 1);
+        int best = 0;
+        size_t best_img = 0;
+        for (int S = smin; S <= smax && S <= p.nsb; S++) {
+            const size_t img = image(S);
+            if (img && (!best || img < best_img)) {
                 best = S;
                 best_img = img;
             }
-            // eight token slots: an image twice the size (the slices' exchange levels cost more than
-            // the waves the larger image takes)
-            const int kib = g_img_kib.load() > 0 ? g_img_kib.load() : MT == 1 ? 20 : 32;
-            if (img <= (size_t)kib * 1024 * (MT == 8 ? 2 : 1)) break;
+            if (img && img <= bound) break;
+        }
+        // One token, short ranges, an image close to the bound: twice the slices where no range then crosses a
+        // slice boundary, one exchange level for half the conversions (us, two slices / four: Q4_K
+        // 17408 x 4096 11.3 / 10.7, x 5120 13.0 / 12.1, Q6_K 15.9 / 15.7; one / two: Q4_K 8192 x 5120 8.75 / 8.45).
+        // Not at 26 KB and less (12288 x 4096 9.08 / 9.29, Q5_K 10.0 / 10.6), nor beyond 100 units a range
+        // (Q5_K 17408 x 17408 36.6 / 37.9), nor for Q8_0, whose longer weight stream covers the conversions
+        // (17408 x 4096 15.2 / 15.9, x 5120 18.2 / 17.8).
+        if (MT == 1 && TYPE != T_Q8_0 && knob == 0 && best && 2 * best <= smax && groups % (2 * best) == 0 &&
+            best_img > 26 * 1024 && p.units <= 100 * groups) {
+            const size_t img = image(2 * best);
+            if (img && img < best_img) best = 2 * best;
         }
         if (!best) return false;
         for (int waves = std::min(g_wpg.load() > 0 ? g_wpg.load() : 16, gemv1_max_waves<MT>()); waves >= 4; waves--) {

@@ -1,0 +1,53 @@
+"""The int8 GEMV's plan (qk_gemv_plan launches nothing, so this runs without a GPU, at 256 CUs): the
+K-slices of a call.
+"""
+import pytest
+
+from oracle_lib import T_Q4_K, T_Q5_K, T_Q6_K, T_Q8_0
+
+TYPES = [T_Q4_K, T_Q5_K, T_Q6_K, T_Q8_0]
+IDS = ["q4k", "q5k", "q6k", "q8_0"]
+FAKE, INT8 = 1 << 20, 1  # an aligned address that nothing reads; QK_GEMV_INT8
+
+
+def _plan(qk, typ, k, ns, m, glu=False, **knobs):
+    try:
+        for name, v in knobs.items():
+            qk.set_tuning(name, v)
+        return qk.gemv_plan([qk.weight_view(FAKE, typ, k, n, 1) for n in ns], glu, m)
+    finally:
+        for name in knobs:
+            qk.set_tuning(name, 0)
+
+
+@pytest.mark.parametrize("typ", TYPES, ids=IDS)
+@pytest.mark.parametrize("k,n", [(6400, 17408), (6656, 5120), (6656, 11888), (7168, 11888), (8960, 11888), (9984, 4096),
+                                 (16640, 5120), (19200, 1600)])
+def test_slices_of_awkward_k(qk, typ, k, n):
+    """Where k / 256 has few divisors a smaller image costs many slices: one token takes no more slices than
+    the 32 KB image bound asks for."""
+    p, bound = _plan(qk, typ, k, [n], 1), _plan(qk, typ, k, [n], 1, gemv_img_kib=32)
+    assert p["kernel"] == INT8 and p["slices"] == bound["slices"]
+
+
+@pytest.mark.parametrize("typ", TYPES, ids=IDS)
+def test_slices_never_jump(qk, typ):
+    """Whatever k and n, one token takes at most one exchange level more than the 32 KB bound, two and four
+    tokens exactly its slices."""
+    for k in range(1024, 19457, 256):
+        for n in (1024, 4096, 5120, 11888, 17408):
+            for m in (1, 2, 4):
+                p, bound = _plan(qk, typ, k, [n], m), _plan(qk, typ, k, [n], m, gemv_img_kib=32)
+                if p["kernel"] != INT8:
+                    continue
+                assert p["slices"] in ((bound["slices"], 2 * bound["slices"]) if m == 1 else (bound["slices"],)), (k, n, m)
+
+
+@pytest.mark.parametrize("typ", TYPES, ids=IDS)
+def test_slices_double_near_the_bound(qk, typ):
+    """One token, k = 17408 and 5120 rows: four slices, each of whose images is half of two slices' (Q8_0 keeps
+    two); 13824, where six slices would cut ranges, keeps the bound's three."""
+    assert _plan(qk, typ, 17408, [5120], 1, gemv_img_kib=32)["slices"] == 2
+    assert _plan(qk, typ, 17408, [5120], 1)["slices"] == (2 if typ == T_Q8_0 else 4)
+    assert _plan(qk, typ, 13824, [5120], 1)["slices"] == _plan(qk, typ, 13824, [5120], 1, gemv_img_kib=32)["slices"]
+    assert _plan(qk, typ, 17408, [17408], 1)["slices"] == 2  # 289 units a range
