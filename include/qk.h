@@ -210,8 +210,8 @@ int qk_gemv_plan(const qk_weight* const* ws, int32_t cnt, int32_t glu, int32_t m
  * the default; 0 = Q4_K / Q6_K through the general kernel, an exact fp16 pair per element of x
  * whose domain is |x| < 65504 with Q4_K 32-element sub-block sums below that too, for comparisons
  * only; Q8_0 / Q5_K always take the int8 kernel),
- * "gemv_wpg" (at most this many waves, 4..16, per int8-kernel work-group; 0 = as many as the LDS
- * holds), "gemv_img_kib" (int8 kernel: the fewest K-slices whose activation image per range fits this
+ * "gemv_wpg" (as many waves per int8-kernel work-group as the LDS holds, at most this many, 4..16;
+ * 0 = the plan's own count, which may be fewer than the LDS holds), "gemv_img_kib" (int8 kernel: the fewest K-slices whose activation image per range fits this
  * many KiB, 1..160; 0 restores the plan's own 32 and its choice of more slices at one token), "gemv_dshift"
  * (int8 kernel: about nu >> value of a work-group's nu units are handed out by a counter, the rest
  * statically; 0..31, default 1), "gemv_min_waves" (int8

@@ -1369,7 +1369,7 @@ int dispatch(int type, int na, int m, F&& f) {
 // data race (which value a concurrent launch sees is unspecified).
 std::atomic<int> g_tune_waves{0};
 std::atomic<bool> g_fused{true};  // m <= 4 through the int8 kernel where its plan applies
-std::atomic<int> g_wpg{0};        // at most this many waves per int8 work-group (0 = as many as fit)
+std::atomic<int> g_wpg{0};        // at most this many waves per int8 work-group (0 = pick_waves)
 std::atomic<int> g_img_kib{0};    // a range's largest activation image before more K-slices (0 = the plan's bound)
 std::atomic<int> g_dshift{1};     // int8 kernel: about nu >> g_dshift of a range's units handed out dynamically
 std::atomic<int> g_min_waves{0};  // int8 kernel at m >= 2: the fewest waves per work-group it is planned with
@@ -1493,23 +1493,43 @@ struct Fused {
         return false;
     }
     // Waves per work-group where the LDS holds w, for ranges of nu units that convert `jobs` (token, super-
-    // block) pairs.  As many as fit is not the fastest: a work-group's waves start ~85 ns apart and a
-    // SIMD with one wave more than the others ends last, so a multiple of four below the most is taken
-    // (us at one token: Q4_K 5120 x 17408 16 waves 12.64, 14 12.8, 12 11.70, 10 12.18, 8 12.46; Q6_K 13 waves
-    // 16.19, 12 15.33, 8 15.36; Q8_0 8192 x 4096 10 waves 9.00, 8 8.71; at four tokens Q4_K 5120 x 5120 16
-    // waves 9.25, 12 8.81), and eight for a range of a few units (Q4_K 1024 x 3072, three units: 16 waves
-    // 6.13, 12 5.55, 8 5.01).  Kept at the most: ranges with more conversions than three a wave (Q4_K
-    // 11008 x 4096, 43: 16 waves 8.93, 12 9.12), many thin slices (Q8_0 11008 x 4096 at two tokens, 43 slices: 11 waves 21.4, 8 24.0), several rounds of
-    // work-groups (Q6_K 5120 x 100000 at two
-    // tokens 11 waves 81.3, 8 84.0) and pairs of two tokens and more, whose unit math is the bound (Q4_K
-    // 5120 x 17408 at four 11 waves 24.9, 8 27.1).
+    // block) pairs.  As many as fit is not always the fastest: a work-group's waves start ~85 ns apart, and a
+    // SIMD with one wave more than the others ends last.  Fitted to 16, 12, 10 and 8 waves at 14 x 15 sizes, four
+    // types and 1, 2 and 4 tokens, checked on 544 random calls that it changes (geometric mean 1.09x the most
+    // waves, nine of them 3..7 % slower).  us, most / chosen:
+    //  * Ranges of a few units: eight (Q4_K 1024 x 3072 at one token, three units: 6.13 / 5.01; up to 15 units at
+    //    one token 1.06x..1.15x, at two where the LDS holds more than twelve).
+    //  * 13..15 waves: twelve, a whole number per SIMD (Q6_K 5120 x 17408 at one 16.2 / 15.3, 11264 x 10192 at two,
+    //    11 slices, 25.3 / 23.9; two rounds, Q4_K 8704 x 13680 at three 30.0 / 27.9).  Kept: many slices at three
+    //    tokens and more (Q5_K 10752 x 3792 at four, 14: 12.5, twelve 14.1).
+    //  * 16 waves: twelve where no wave then converts more often (Q4_K 5120 x 17408 at one 12.6 / 11.7), and where
+    //    one conversion a wave becomes two at one and two tokens (Q4_K 4096 x 8192 7.3 / 6.9) or two become
+    //    three in ranges short or long enough not to wait for them.  Kept: more conversions (Q4_K 7168 x 6144, 28
+    //    of them: 8.40, twelve 8.68; at four tokens 5120 x 11008 13.9, twelve 14.6) and ranges that give twelve
+    //    waves two or three whole units each, the last to start ending last (Q5_K 6144 x 4096 7.2, twelve 7.6).
+    //  * 9..11 waves: eight only in short ranges without more conversions a wave (Q8_0 8192 x 4096 at one
+    //    9.0 / 8.7) and few slices (Q8_0 5376 x 5408 at four, seven: 11.2, eight 12.4); long ranges need them all
+    //    (Q5_K 16384 x 17408 at two 36.8, eight 44.4; Q4_K 7168 x 32000 at four 35.7, eight 42.5).
+    // All of them: many thin slices (Q6_K 11008 x 12288 at two, 43: 45.9, twelve 47.3), 9..11 in several rounds of
+    // work-groups (Q6_K 5120 x 100000 at two 81.3, eight 84.0), pairs of two tokens and more, whose unit math is
+    // the bound (Q4_K 5120 x 17408 at four 24.9, eight 27.1).
     static int pick_waves(int w, int S, int nu, int jobs, bool one_round) {
         if (MT == 8 || (NA == 2 && MT > 1)) return w;
-        if (jobs <= 36 && S <= 8 && one_round) {
-            if (nu < 16) return std::min(w, 8);
-            return w >= 12 ? 12 : w >= 8 ? 8 : w;
+        if (!one_round) return w > 12 && w < 16 ? 12 : w;
+        auto passes = [&](int waves) { return (jobs + waves - 1) / waves; };  // conversions of the busiest wave
+        if (nu <= 8 || (MT == 1 && S <= 8 && nu < 16)) return std::min(w, 8);
+        if (w <= 12) {
+            const int longest = MT == 4 ? 64 : MT == 2 ? 24 : 36;
+            const bool eight = (passes(8) == passes(w) && nu <= longest) || (MT == 1 && nu <= 24);
+            return w > 8 && w < 12 && S <= 4 && eight ? 8 : w;
         }
-        return w > 12 && w < 16 ? 12 : w;
+        if (S > 8) return w < 16 && S <= 16 && MT <= 2 ? 12 : w;
+        if (MT == 2 && nu < 16) return 8;
+        if (w < 16) return 12;
+        const int p = passes(16);
+        if (passes(12) == p) return nu == 23 || nu == 24 || (nu >= 33 && nu <= 36) ? w : 12;
+        if (p == 1) return MT <= 2 || S == 1 ? 12 : w;
+        return p == 2 && (nu <= 20 || (MT <= 2 && nu > 45)) ? 12 : w;
     }
     // Plan for `groups` work-groups: the fewest slices (from smin, at most smax) whose range image fits 32 KB
     // (64 with eight token slots: the slices' exchange levels cost more than the waves the larger image

@@ -81,7 +81,7 @@ constexpr int MAX_DEVICES = 64;
 int gemv_plan_waves(int type, int na, int m, int units);
 void gemv_set_waves(int waves);  // tuning override of the plan (0 = occupancy-derived)
 void gemv_set_fused(bool on);    // m == 1 through the single-token kernel (default on)
-void gemv_set_wpg(int w);        // single-token kernel: cap on waves per work-group (0 = LDS-limited)
+void gemv_set_wpg(int w);        // single-token kernel: cap on waves per work-group (0 = planned)
 void gemv_set_img_kib(int kib);  // int8 kernel: activation image per range before more K-slices (0 = the plan's bound)
 void gemv_set_dshift(int sh);    // int8 kernel: about nu >> sh of a range's units handed out dynamically
 void gemv_set_min_waves(int w);  // int8 kernel at m >= 2: fewest waves per work-group (else the general kernel)

@@ -1,5 +1,5 @@
 """The int8 GEMV's plan (qk_gemv_plan launches nothing, so this runs without a GPU, at 256 CUs): the
-K-slices of a call.
+K-slices and the waves of a call.
 """
 import pytest
 
@@ -51,3 +51,18 @@ def test_slices_double_near_the_bound(qk, typ):
     assert _plan(qk, typ, 17408, [5120], 1)["slices"] == (2 if typ == T_Q8_0 else 4)
     assert _plan(qk, typ, 13824, [5120], 1)["slices"] == _plan(qk, typ, 13824, [5120], 1, gemv_img_kib=32)["slices"]
     assert _plan(qk, typ, 17408, [17408], 1)["slices"] == 2  # 289 units a range
+
+
+@pytest.mark.parametrize("typ,k,n,m", [(T_Q5_K, 16384, 17408, 2), (T_Q5_K, 4096, 76016, 2), (T_Q4_K, 7168, 32000, 4),
+                                       (T_Q6_K, 9216, 6144, 4), (T_Q8_0, 7168, 12288, 1), (T_Q4_K, 7168, 5120, 3)])
+def test_waves_kept(qk, typ, k, n, m):
+    """Calls that a smaller work-group slows down run as many waves as the LDS holds."""
+    p, most = _plan(qk, typ, k, [n], m), _plan(qk, typ, k, [n], m, gemv_wpg=16)
+    assert p["kernel"] == INT8 and p["waves_per_group"] == most["waves_per_group"] > 8 and p["slices"] == most["slices"]
+
+
+@pytest.mark.parametrize("typ,k,n,m,waves", [(T_Q4_K, 1024, 3072, 1, 8), (T_Q4_K, 5120, 17408, 1, 12), (T_Q6_K, 5120, 17408, 1, 12),
+                                             (T_Q8_0, 6144, 5120, 1, 8), (T_Q4_K, 5120, 5120, 4, 12)])
+def test_waves_reduced(qk, typ, k, n, m, waves):
+    """Calls that run on fewer: short ranges on eight, others on a whole number per SIMD."""
+    assert _plan(qk, typ, k, [n], m)["waves_per_group"] == waves < _plan(qk, typ, k, [n], m, gemv_wpg=16)["waves_per_group"]
