@@ -1429,7 +1429,7 @@ struct Fused {
         p.lds_ring = (int)align16(p.lds_tab + 16 * (size_t)maxnu);
         return p.lds_ring + (size_t)waves * D * NA * C::GB;
     }
-    static bool plan(GemvParams& p, int cus, bool small, int& wpg, size_t& lds) {
+    static bool plan(GemvParams& p, int cus, bool small, int min_waves, int& wpg, size_t& lds) {
         // one work-group per CU; more (smaller ranges, run in rounds) when one range's tables do not
         // fit the LDS, or leave it room for fewer than WANT waves: a range's unit sums and table grow
         // with its units (a 248320-row matrix left four waves per CU at one work-group per CU, and
@@ -1444,7 +1444,7 @@ struct Fused {
             GemvParams t = p;
             int w = 0;
             size_t l = 0;
-            if (plan_groups(t, groups, groups <= cus, MT == 8 ? 32 : 16, w, l) && w > best_w) {
+            if (plan_groups(t, groups, groups <= cus, min_waves, MT == 8 ? 32 : 16, w, l) && w > best_w) {
                 best = t;
                 best_w = w;
                 best_lds = l;
@@ -1485,7 +1485,7 @@ struct Fused {
         for (int ci = 0; ci < nc; ci++) {
             const Cand& c = cands[ci];
             GemvParams t = p;
-            if (plan_groups(t, c.g, true, c.S, wpg, lds, c.S)) {
+            if (plan_groups(t, c.g, true, min_waves, c.S, wpg, lds, c.S)) {
                 p = t;
                 return true;
             }
@@ -1537,7 +1537,8 @@ struct Fused {
     // slices where they have few divisors (one token, 20 KB against 32, us: Q4_K 6656 x 11888 13 slices 16.1, one
     // 11.4; 9984 x 5120 13 slices 12.7, three 10.0; 6400 x 17408 five slices 16.7, one 13.9; Q5_K, Q6_K and Q8_0
     // alike); the knob gemv_img_kib sets another.
-    static bool plan_groups(GemvParams& p, int groups, bool one_round, int smax, int& wpg, size_t& lds, int smin = 1) {
+    static bool plan_groups(GemvParams& p, int groups, bool one_round, int min_waves, int smax, int& wpg, size_t& lds,
+                            int smin = 1) {
         const int ntiles = p.units / p.nsb;
         auto image = [&](int S) -> size_t {  // of the largest range; 0 when S slices are not possible
             GemvParams t = p;
@@ -1577,8 +1578,9 @@ struct Fused {
                 wpg = waves;
                 lds = total;
                 if (g_wpg.load() == 0) {
-                    const int w = pick_waves(waves, best, (p.units + groups - 1) / groups, t.lds_part / G1<TYPE, MT>::IMG * MT,
-                                             one_round);
+                    const int picked = pick_waves(waves, best, (p.units + groups - 1) / groups,
+                                                  t.lds_part / G1<TYPE, MT>::IMG * MT, one_round);
+                    const int w = std::max(picked, std::min(min_waves, waves));  // the knob counts what the LDS holds
                     GemvParams f = p;
                     if (const size_t fewer = w < waves ? layout(f, groups, best, w) : 0) {
                         t = f;
@@ -1605,7 +1607,7 @@ struct Fused {
         int wpg = 0;
         size_t lds = 0;
         // not applicable: the caller uses the general kernel
-        if (!plan(p, cus, small, wpg, lds) || wpg < min_waves) return 1;
+        if (!plan(p, cus, small, min_waves, wpg, lds) || wpg < min_waves) return 1;
         if (info) {
             info->kernel = GEMV_KERNEL_INT8;
             info->work_groups = p.waves;

@@ -66,3 +66,18 @@ def test_waves_kept(qk, typ, k, n, m):
 def test_waves_reduced(qk, typ, k, n, m, waves):
     """Calls that run on fewer: short ranges on eight, others on a whole number per SIMD."""
     assert _plan(qk, typ, k, [n], m)["waves_per_group"] == waves < _plan(qk, typ, k, [n], m, gemv_wpg=16)["waves_per_group"]
+
+
+@pytest.mark.parametrize("typ", [T_Q4_K, T_Q6_K], ids=["q4k", "q6k"])
+@pytest.mark.parametrize("m", [2, 4])
+def test_min_waves_counts_what_the_lds_holds(qk, typ, m):
+    """gemv_min_waves sends a call to the general kernel where the LDS holds fewer waves than it asks for, not
+    where the plan takes fewer than the LDS holds."""
+    k = n = 5120
+    held = _plan(qk, typ, k, [n], m, gemv_wpg=16)["waves_per_group"]
+    assert _plan(qk, typ, k, [n], m)["waves_per_group"] == 12 < held
+    for w in (12, held):
+        p = _plan(qk, typ, k, [n], m, gemv_min_waves=w)
+        assert p["kernel"] == INT8 and w <= p["waves_per_group"] <= held
+    if held < 16:
+        assert _plan(qk, typ, k, [n], m, gemv_min_waves=held + 1)["kernel"] != INT8
