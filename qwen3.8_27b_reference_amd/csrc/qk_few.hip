@@ -278,9 +278,12 @@ int launch_few_type(const FewParams& p, size_t lds, hipStream_t s) {
 
 }  // namespace
 
-// Plan: the K-slices of least estimated time (us), from sweeps of every slice count on 7 shapes at 8 and 13
-// tokens: the busiest CU's units at 24 KB/us, its image of x at 60 KB/us, 3 us for the sum's launch and
-// 0.9 us per MB of partials (each part written, then read), 1.2 us where tiles are cut between waves.
+// Plan: the K-slices of least estimated time (us), fitted to every slice count with 8 and 12 waves on 50 sizes of
+// the four types at 5 and 13 tokens, single and as gate/up pairs (the slices chosen are 1.1 % slower than the best
+// in the geometric mean, 13 % at most): the busiest CU's units at 24 KB/us, its image of x at 50 KB/us, 1.1 us where
+// a tile is cut between waves, and for the second launch 1.7 us, 1.1 us per MB of partials (each part written, then
+// read) and 1.1 us for the parts its threads load together (four; a single matrix's of more than four, eight): a
+// pair of 8192 x 512 at 5 tokens in 32 slices took 13.7 us, in four 8.4.
 // Eight waves (two per SIMD) with two units each in flight beat every larger ring on every shape (Q6_K
 // 17408 x 5120 at 13 tokens: 8 waves x 2 units 20.4 us, 8 x 3 21.4, 12 x 2 21.3, 16 x 3 24.1; Q4_K 5120 x 17408
 // at 8 tokens 15.4 / 15.6 / 15.3 / 18.9); twelve where a CU has many units (the gate/up pair of 5120 x 17408
@@ -297,8 +300,11 @@ bool few_plan(int type, FewParams& p, int cus, size_t rows, size_t part_cap, boo
         int waves = units >= 128 ? 12 : 8;
         if (img + (size_t)waves * DEPTH * gb > LDS_PER_CU) waves = 8;
         if (img + (size_t)waves * DEPTH * gb > LDS_PER_CU || units * waves >= (1ll << 31)) continue;
-        const double t = units * gb / 24e3 + cs * xsb / 60e3 + (tiles % waves ? 1.2 : 0.0) +
-                         (parts ? 3.0 + S * 4.0 * p.m * (double)rows * 0.9e-6 : 0.0);
+        bool cut = false;  // a wave of the largest range starts inside a tile
+        for (int w = 1; w < waves; w++) cut |= w * units / waves % cs != 0;
+        const int loads = sums ? (S + 3) / 4 : S <= 4 ? 1 : (S + 7) / 8 * 2;
+        const double t = units * gb / 24e3 + cs * xsb / 50e3 + (cut ? 1.1 : 0.0) +
+                         (parts ? 1.7 + S * 4.0 * p.m * (double)rows * 1.1e-6 + 1.1 * loads : 0.0);
         if (best == 0.0 || t < best) {
             best = t;
             p.slices = S;
