@@ -288,8 +288,18 @@ int launch_few_type(const FewParams& p, size_t lds, hipStream_t s) {
 // 17408 x 5120 at 13 tokens: 8 waves x 2 units 20.4 us, 8 x 3 21.4, 12 x 2 21.3, 16 x 3 24.1; Q4_K 5120 x 17408
 // at 8 tokens 15.4 / 15.6 / 15.3 / 18.9); twelve where a CU has many units (the gate/up pair of 5120 x 17408
 // at 13 tokens 26.4 -> 25.8).
+// No plan, so the GEMM, for Q4_K and Q8_0 beyond eight tokens where its work-groups of eight tile pairs fill 93 %
+// and more of whole rounds of the CUs and a tile holds 36 KB: there its one barrier a step is hidden and its
+// activations need no image (us, this kernel / the GEMM at 16 tokens: Q4_K 4096 x 128256 68.5 / 58.9, 4096 x 65536
+// 36.3 / 33.0, Q8_0 3072 x 65536 44.6 / 40.5; over k = 4096..8192 and 65536, 128256 and 248320 rows at 9, 12 and 16 tokens
+// the GEMM is 1.06x for both types).  Below the lines this kernel is ahead: rounds of 77 %, Q4_K 4096 x 151936
+// 1.03x..1.24x, tiles of 28 KB, Q4_K 3072 x 65536 1.03x..1.14x, eight tokens 1.06x, Q5_K 1.17x, Q6_K 1.34x.
 bool few_plan(int type, FewParams& p, int cus, size_t rows, size_t part_cap, bool sums, size_t& lds) {
     const int gb = group_bytes(type), xsb = XREC * (p.m <= 8 ? 8 : 16) * 16;
+    if ((type == T_Q4_K || type == T_Q8_0) && p.m > 8 && p.cnt == 1 && !sums && p.nsb * gb >= 36000) {
+        const long long wgs = (p.ntiles + 15) / 16, rounds = (wgs + cus - 1) / cus;
+        if (100 * wgs >= 93 * rounds * cus) return false;
+    }
     double best = 0.0;
     for (int S = 1; S <= p.nsb && S <= cus && S <= MAX_SLICES; S++) {
         const bool parts = S > 1 || sums;

@@ -945,10 +945,12 @@ int launch_ntb(const GemmCall& c) {
 }
 
 // Up to 16 tokens: the weight-streaming form (qk_few.hip), where it has a plan and no knob asks for a plan
-// of this kernel.  Measured against this kernel at 5, 8, 13 and 16 tokens on 17 shapes: faster on every
-// one (us at 13 tokens: Q4_K 17408 x 5120 19.8 -> 16.8, Q6_K 27.1 -> 21.3, Q5_K 23.0 -> 20.0, Q8_0 6144 x 5120
-// 15.1 -> 12.4, the gate/up pair of 5120 x 17408 34.7 -> 26.6, the output projection 272 -> 214; least
-// gain Q4_K 1024 x 3072 x 2 7.9 -> 7.6).  Its x image has 16 token columns: above, this kernel's 32.
+// of this kernel.  Over 1332 calls at 5, 8, 12 and 16 tokens (groups and gate/up pairs to 15) it takes 1 / 1.28 of this
+// kernel's time in the geometric mean (us at 13 tokens: Q4_K 17408 x 5120 19.8 -> 16.8, Q6_K 27.1 -> 21.3, Q5_K
+// 23.0 -> 20.0, Q8_0 6144 x 5120 15.1 -> 12.4, the gate/up pair of 5120 x 17408 34.7 -> 26.6, the output projection
+// 272 -> 214).  few_plan leaves the calls whose rounds this kernel fills; what stays slower on it are some Q8_0
+// calls of 60 MB and more whose K-parts fill a round here (pair 3072 x 10240 at 8 tokens 18.3 -> 21.5, 3072 x 32000 at 16
+// 20.1 -> 24.0), where neither plan's estimate tells which.  Its x image has 16 token columns: above, this kernel's 32.
 // Returns 1 when it does not take the call.
 template <int TYPE>
 int launch_few_call(const GemmCall& c) {

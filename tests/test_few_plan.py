@@ -49,3 +49,12 @@ def test_plans_fit(qk, typ):
                     assert lds <= 160 * 1024 and p.waves in (8, 12) and 1 <= p.slices * p.wgs <= 256
                     assert p.wgs <= p.ntiles and p.slices <= k // 256
                     assert (p.slices == 1 and len(ns) != 2) or p.slices * m * sum(ns) <= cap
+
+
+@pytest.mark.parametrize("typ,k,n,m,few", [(T_Q4_K, 4096, 65536, 16, False), (T_Q4_K, 8192, 128256, 9, False), (T_Q8_0, 3072, 65536, 12, False),
+                                           (T_Q4_K, 4096, 65536, 8, True), (T_Q4_K, 3072, 65536, 16, True),
+                                           (T_Q4_K, 4096, 151936, 16, True), (T_Q5_K, 4096, 65536, 16, True),
+                                           (T_Q6_K, 5120, 248320, 13, True)])
+def test_whole_gemm_rounds(qk, typ, k, n, m, few):
+    """Q4_K and Q8_0 beyond eight tokens leave calls that fill whole rounds of the GEMM's work-groups to it."""
+    assert (_plan(qk, typ, k, [n], m)[0] is not None) == few
