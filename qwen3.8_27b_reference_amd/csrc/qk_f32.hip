@@ -7,8 +7,8 @@
 // The matrices are small (5120 x 48 in the model), so what bounds a call is how many CUs its loads
 // are spread over, not the bytes.  Two kernels, both without a workspace (F32 calls need none, so they
 // may come first on a stream under capture):
-//  * k_f32_rows: one work-group per 1, 2 or 4 rows, k split over its 256 threads, up to 16 tokens per
-//    pass.  n = 48, k = 5120 (us per call, graph-timed, one wave per row before): one token 10.4 ->
+//  * k_f32_rows: one work-group per 1, 2 or 4 rows, k split over its 256 threads (rows of up to 768 elements:
+//    over a wave), up to 16 tokens per pass.  n = 48, k = 5120 (us per call, graph-timed, one wave per row before): one token 10.4 ->
 //    2.6 (~2 of them the launch), 13 tokens 66 -> 3.3, 512 tokens 3540 -> 12.3.
 //  * k_f32_tile: fp32 MFMA on tiles of 16 x 16 or 32 x 32 (rows x tokens), k split over the sixteen waves of the
 //    work-group, their sums added through LDS in wave order.  n = 1024, m = 512 58 us (93 TFLOP/s);
@@ -45,15 +45,17 @@ struct X8 {
 // Sum over the wave's 64 lanes on the VALU (every lane gets it).
 __device__ inline float wave_sum(float v) { return xor32_sum(xor16_sum(sum16(v))); }
 
-// Rows RW * blockIdx.x .. + RW - 1 of matrix blockIdx.z for tokens MT * blockIdx.y .. + MT - 1 (rows and
-// tokens past the ends re-read the last one and are not stored).  Thread i takes elements 4 i ..
-// 4 i + 3 of every 1024.
-template <int FMT, int RW, int MT>
+// Tokens MT * blockIdx.y .. + MT - 1 of rows of matrix blockIdx.z (rows and tokens past the ends re-read the last
+// one and are not stored), RW rows at a time with k over KT threads.
+// KT = 256: the work-group's rows are RW * blockIdx.x .. + RW - 1; thread i takes elements 4 i .. 4 i + 3 of every
+// 1024.  KT = 64: each wave has RW rows of its own and thread i elements 4 i .. of every 256, for rows too
+// short to occupy 256 threads.
+template <int FMT, int RW, int MT, int KT>
 __global__ __launch_bounds__(256) void k_f32_rows(const F32Mats M, int k, const void* __restrict__ x, int m) {
-    const int z = blockIdx.z, n = M.n[z], row0 = blockIdx.x * RW, t0 = blockIdx.y * MT;
-    if (row0 >= n) return;
-    __shared__ float part[4][RW * MT];
-    const int tid = threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int z = blockIdx.z, n = M.n[z], t0 = blockIdx.y * MT;
+    const int row0 = KT == 256 ? blockIdx.x * RW : (blockIdx.x * 4 + wave) * RW;
+    if (row0 >= n) return;  // KT = 64: no barrier follows
     const float* wr[RW];
 #pragma unroll
     for (int i = 0; i < RW; i++) wr[i] = M.w[z] + (size_t)min(row0 + i, n - 1) * k;
@@ -62,9 +64,10 @@ __global__ __launch_bounds__(256) void k_f32_rows(const F32Mats M, int k, const 
     for (int i = 0; i < RW; i++)
 #pragma unroll
         for (int t = 0; t < MT; t++) acc[i][t] = 0.0f;
-    constexpr int U = MT == 1 ? 5 : MT == 4 && RW == 1 ? 2 : 1;  // passes whose loads go out together
+    // passes whose loads go out together
+    constexpr int U = KT == 64 ? 1 : MT == 1 ? 5 : MT == 4 && RW == 1 ? 2 : 1;
 #pragma unroll U
-    for (int e = 4 * tid; e < k; e += 1024) {
+    for (int e = 4 * (KT == 256 ? threadIdx.x : lane); e < k; e += 4 * KT) {
         f4 wv[RW], xv[MT];
 #pragma unroll
         for (int i = 0; i < RW; i++) wv[i] = *(const f4*)(wr[i] + e);
@@ -76,18 +79,33 @@ __global__ __launch_bounds__(256) void k_f32_rows(const F32Mats M, int k, const 
             for (int t = 0; t < MT; t++)
                 acc[i][t] = fmaf(wv[i].x, xv[t].x, fmaf(wv[i].y, xv[t].y, fmaf(wv[i].z, xv[t].z, fmaf(wv[i].w, xv[t].w, acc[i][t]))));
     }
+    // sum t RW + i: over the wave's lanes, and over the four waves where they share a row
+    float sum = 0.0f;
+    int o = lane;
+    if constexpr (KT == 256) {
+        __shared__ float part[4][RW * MT];
 #pragma unroll
-    for (int i = 0; i < RW; i++)
+        for (int i = 0; i < RW; i++)
 #pragma unroll
-        for (int t = 0; t < MT; t++) {
-            const float v = wave_sum(acc[i][t]);
-            if ((tid & 63) == 0) part[tid >> 6][t * RW + i] = v;
-        }
-    __syncthreads();
-    if (tid < RW * MT) {
-        const int t = t0 + tid / RW, row = row0 + tid % RW;
-        if (row < n && t < m) M.y[z][(size_t)t * n + row] = (part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]);
+            for (int t = 0; t < MT; t++) {
+                const float v = wave_sum(acc[i][t]);
+                if (lane == 0) part[wave][t * RW + i] = v;
+            }
+        __syncthreads();
+        o = threadIdx.x;
+        if (o < RW * MT) sum = (part[0][o] + part[1][o]) + (part[2][o] + part[3][o]);
+    } else {
+        static_assert(RW * MT <= 64, "a lane per sum");
+#pragma unroll
+        for (int i = 0; i < RW; i++)
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                const float v = wave_sum(acc[i][t]);
+                if (lane == t * RW + i) sum = v;
+            }
     }
+    const int t = t0 + o / RW, row = row0 + o % RW;
+    if (o < RW * MT && row < n && t < m) M.y[z][(size_t)t * n + row] = sum;
 }
 
 // D(16x16 f32) += A(16x4 f32) * B(4x16 f32).  Lane l holds A[l & 15][l >> 4], B[l >> 4][l & 15] and
@@ -159,10 +177,11 @@ __global__ __launch_bounds__(64 * TILE_WAVES) void k_f32_tile(const F32Mats M, i
 
 constexpr int MAX_GRID_Y = 65535;
 
-template <int FMT, int RW, int MT>
+template <int FMT, int RW, int MT, int KT = 256>
 void launch_rows(const F32Mats& M, int nmax, int cnt, int k, const void* x, int m, hipStream_t s) {
-    hipLaunchKernelGGL((k_f32_rows<FMT, RW, MT>), dim3((nmax + RW - 1) / RW, (m + MT - 1) / MT, cnt), dim3(256), 0, s, M,
-                       k, x, m);
+    constexpr int ROWS = RW * (256 / KT);
+    hipLaunchKernelGGL((k_f32_rows<FMT, RW, MT, KT>), dim3((nmax + ROWS - 1) / ROWS, (m + MT - 1) / MT, cnt), dim3(256), 0, s,
+                       M, k, x, m);
 }
 template <int FMT, int R>
 void launch_tile(const F32Mats& M, int nmax, int cnt, int k, const void* x, int m, hipStream_t s) {
@@ -195,14 +214,23 @@ void launch_fmt(const F32Mats& M, int cnt, int k, const void* x, int m, hipStrea
     //    against 12.3).
     //  * Rows share the loads of x as soon as the work-groups left still cover the CUs (n = 48: m = 16 one
     //    row 3.29, two 3.78; m = 64 4.50 / 4.41 / four 4.61; m = 256 10.8 / 7.9 / 7.25).
+    //  * Rows of up to 768 elements leave a quarter and more of 256 threads without any: a wave per two or four rows
+    //    where a call has enough of them to fill the CUs (us, one wave per row / 256 threads / this: k = 256, n =
+    //    65536, m = 1 19.2 / 25.3 / 11.1, m = 5 40.3 / 47.7 / 17.2, m = 13 81.2 / 110 / 33.2; n = 4096, m = 5 5.5 /
+    //    5.1 / 3.6; k = 768, n = 65536, m = 1 36.1 / 41.4 / 34.0; at k = 1024 44.9 / 43.2 / 45.5).
     // (Past 2^23 rows a work-group per row would exceed a grid's 2^32 threads.)
     if ((m > 16 && rows * m >= 96 * 1024) || nmax > (1 << 23)) return launch_tile<FMT, 2>(M, nmax, cnt, k, x, m, s);
     long long tiles = 0;
     for (int z = 0; z < cnt; z++) tiles += (long long)((M.n[z] + 15) / 16) * ((m + 15) / 16);
     if (rows * m >= 44 * 1024 && tiles <= 256) return launch_tile<FMT, 1>(M, nmax, cnt, k, x, m, s);
+    const long long passes = rows * ((m + 3) / 4);
+    if (k <= 768 && passes >= 4096) {
+        if (m == 1) return launch_rows<FMT, 2, 1, 64>(M, nmax, cnt, k, x, m, s);
+        if (m <= 4) return launch_rows<FMT, 2, 4, 64>(M, nmax, cnt, k, x, m, s);
+        return launch_rows<FMT, 4, 8, 64>(M, nmax, cnt, k, x, m, s);
+    }
     if (m == 1) return launch_rows<FMT, 1, 1>(M, nmax, cnt, k, x, m, s);
     if (m > 8 && m <= 16 && rows * k > (8ll << 20)) return launch_rows<FMT, 4, 16>(M, nmax, cnt, k, x, m, s);
-    const long long passes = rows * ((m + 3) / 4);
     if (m > 4 && passes >= 8192) return launch_rows<FMT, 4, 8>(M, nmax, cnt, k, x, m, s);
     if (passes >= 2048) return launch_rows<FMT, 4, 4>(M, nmax, cnt, k, x, m, s);
     if (passes >= 512) return launch_rows<FMT, 2, 4>(M, nmax, cnt, k, x, m, s);

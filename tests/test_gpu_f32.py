@@ -33,6 +33,8 @@ def _weights(n, k, seed):
 SHAPES = [(256, 1, 1), (1280, 3, 2), (5120, 48, 4), (768, 5, 5), (256, 17, 9), (5120, 48, 13), (1024, 130, 17),
           (1280, 127, 22), (256, 1031, 8), (1024, 2050, 15), (256, 4099, 6), (8448, 1030, 13), (256, 97, 1025),
           (1280, 1601, 63), (768, 33, 3001),
+          # a wave per two or four rows (k <= 768, many rows), ragged rows and tokens, one past its longest k
+          (256, 4097, 1), (512, 5003, 3), (768, 1027, 16), (256, 2052, 7), (512, 1500, 11), (768, 4099, 1), (1024, 4099, 1),
           # 16 x 16 tiles: at 256 tiles and one past, ragged rows and tokens, on the line of 44 Ki outputs
           (1280, 4096, 11), (256, 4091, 16), (768, 4097, 13), (2304, 44, 1024), (256, 47, 1013), (5120, 241, 255)]
 
