@@ -22,8 +22,10 @@ namespace {
 // fall into different banks.
 // Bound: HBM, each byte read and written once.  Measured (us, GGUF -> T16 / back; one byte per thread and
 // access before): Q4_K 5120 x 17408 60.8 -> 18.9 (5.3 TB/s) / 62.5 -> 21.5, Q6_K 17408 x 5120 103.5 -> 34.6 /
-// 119.8 -> 46.1, Q6_K 5120 x 248320 1460 -> 378 / 1636 -> 459.  Smaller chunks, down to one super-block where
-// the tiles are few, measured the same or slower (Q8_0 6144 x 5120 14.4 -> 15.6 at 1024 work-groups).
+// 119.8 -> 46.1, Q6_K 5120 x 248320 1460 -> 378 / 1636 -> 459.  A chunk is 1, 2, 4 or 8 super-blocks, the fewest
+// that leave at most 1152 work-groups: smaller tensors are bound by one chunk's time (Q6_K 17408 x 48 to GGUF in
+// chunks of 8, 4, 2, 1: 10.1 7.3 4.7 4.0, a byte per thread before 6.4; x 512 12.4 9.6 7.8 9.1; 6144 x 1024 10.2 8.6 6.4
+// 7.7), larger ones by the words that a window shares with its neighbours (17408 x 5120 42.4 44.7 48.4 66.2).
 constexpr int REPACK_SBS = 8;
 template <int TYPE>
 struct Repack {
@@ -354,7 +356,9 @@ __global__ __launch_bounds__(256) void k_synth(uint8_t* __restrict__ dst, int ty
 
 template <int TYPE>
 static void launch_repack_type(const uint8_t* src, uint8_t* dst, int nsb, int n, int dir, hipStream_t s) {
-    const dim3 grid((nsb + REPACK_SBS - 1) / REPACK_SBS, n / 16);
+    int sbs = 1;  // super-blocks per chunk, see REPACK_SBS
+    while (sbs < REPACK_SBS && (long long)nsb * (n / 16) > 1152ll * sbs) sbs *= 2;
+    const dim3 grid((nsb + sbs - 1) / sbs, n / 16);
     if (dir == 0) hipLaunchKernelGGL((k_repack<TYPE, true>), grid, dim3(256), 0, s, src, dst, nsb);
     else hipLaunchKernelGGL((k_repack<TYPE, false>), grid, dim3(256), 0, s, src, dst, nsb);
 }

@@ -10,7 +10,9 @@ from oracle_lib import SEED_BASE, T_Q4_K, T_Q5_K, T_Q6_K, T_Q8_0
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(256, 16), (512, 48), (2048, 32), (2304, 16), (4352, 80), (5120, 272), (17408, 16), (7936, 400)]
+SHAPES = [(256, 16), (512, 48), (2048, 32), (2304, 16), (4352, 80), (5120, 272), (17408, 16), (7936, 400),
+          # chunks of two, four and eight super-blocks (the shapes above: one)
+          (4352, 1360), (7936, 1600), (5888, 6400)]
 GUARD = 256
 
 
