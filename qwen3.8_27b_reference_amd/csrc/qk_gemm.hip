@@ -740,7 +740,12 @@ __device__ inline f4 sum_parts(const f4* __restrict__ part, size_t stride, int k
     return v;
 }
 
-// Adds the ks partial results [ks][m][n] of matrix blockIdx.y in part order (deterministic) into its y.
+// Adds the ks partial results [ks][m][n] of matrix blockIdx.y in part order (deterministic) into its y.  Outputs of
+// 576 and more work-groups hide the loads' latency themselves and are faster one part after another (us of a whole
+// call, several in flight / one: Q4_K 6144 x 1024 at 640 tokens 28.6 / 28.0, 5120 x 5120 at 128 23.9 / 22.8, Q6_K 17408 x
+// 2048 at 512 60.4 / 59.5; fewer work-groups: Q4_K 5120 x 1024 at 100 12.3 / 13.1, 17408 x 5120 at 48 24.5 / 25.3, equal
+// at 500).
+constexpr size_t SUM_SERIAL = 576 * 256;
 struct SumMats {
     const f4* part[GEMM_MATS];
     f4* y[GEMM_MATS];
@@ -753,7 +758,8 @@ __global__ __launch_bounds__(256) void k_splitk_sum(const SumMats S, int ks) {
     const size_t n4 = S.n4[blockIdx.y];
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) {
         const size_t o = S.ldy4 ? i / S.n4row * S.ldy4 + i % S.n4row : i;
-        y[o] = ks <= 4 ? sum_parts<4>(part + i, n4, ks) : sum_parts<8>(part + i, n4, ks);
+        y[o] = n4 >= SUM_SERIAL ? sum_parts<1>(part + i, n4, ks)
+               : ks <= 4 ? sum_parts<4>(part + i, n4, ks) : sum_parts<8>(part + i, n4, ks);
     }
 }
 
