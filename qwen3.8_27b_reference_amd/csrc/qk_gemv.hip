@@ -1501,15 +1501,17 @@ struct Fused {
     //    one token 1.06x..1.15x, at two where the LDS holds more than twelve).
     //  * 13..15 waves: twelve, a whole number per SIMD (Q6_K 5120 x 17408 at one 16.2 / 15.3, 11264 x 10192 at two,
     //    11 slices, 25.3 / 23.9; two rounds, Q4_K 8704 x 13680 at three 30.0 / 27.9).  Kept: many slices at three
-    //    tokens and more (Q5_K 10752 x 3792 at four, 14: 12.5, twelve 14.1).
+    //    tokens and more (Q5_K 10752 x 3792 at four, 14: 12.5, twelve 14.1) and of short ranges (Q6_K 6656 x 4256
+    //    at two, 13: 10.8, twelve 11.8).
     //  * 16 waves: twelve where no wave then converts more often (Q4_K 5120 x 17408 at one 12.6 / 11.7), and where
     //    one conversion a wave becomes two at one and two tokens (Q4_K 4096 x 8192 7.3 / 6.9) or two become
     //    three in ranges short or long enough not to wait for them.  Kept: more conversions (Q4_K 7168 x 6144, 28
     //    of them: 8.40, twelve 8.68; at four tokens 5120 x 11008 13.9, twelve 14.6) and ranges that give twelve
     //    waves two or three whole units each, the last to start ending last (Q5_K 6144 x 4096 7.2, twelve 7.6).
     //  * 9..11 waves: eight only in short ranges without more conversions a wave (Q8_0 8192 x 4096 at one
-    //    9.0 / 8.7) and few slices (Q8_0 5376 x 5408 at four, seven: 11.2, eight 12.4); long ranges need them all
-    //    (Q5_K 16384 x 17408 at two 36.8, eight 44.4; Q4_K 7168 x 32000 at four 35.7, eight 42.5).
+    //    9.0 / 8.7) and few slices (Q8_0 5376 x 5408 at four, seven: 11.2, eight 12.4); pairs beyond 15 units
+    //    (Q4_K 2048 x 13312 9.0, eight 9.5) and long ranges need them all (Q5_K 16384 x 17408 at two 36.8, eight
+    //    44.4; Q4_K 7168 x 32000 at four 35.7, eight 42.5).
     // All of them: many thin slices (Q6_K 11008 x 12288 at two, 43: 45.9, twelve 47.3), 9..11 in several rounds of
     // work-groups (Q6_K 5120 x 100000 at two 81.3, eight 84.0), pairs of two tokens and more, whose unit math is
     // the bound (Q4_K 5120 x 17408 at four 24.9, eight 27.1).
@@ -1521,9 +1523,9 @@ struct Fused {
         if (w <= 12) {
             const int longest = MT == 4 ? 64 : MT == 2 ? 24 : 36;
             const bool eight = (passes(8) == passes(w) && nu <= longest) || (MT == 1 && nu <= 24);
-            return w > 8 && w < 12 && S <= 4 && eight ? 8 : w;
+            return w > 8 && w < 12 && S <= 4 && NA == 1 && eight ? 8 : w;
         }
-        if (S > 8) return w < 16 && S <= 16 && MT <= 2 ? 12 : w;
+        if (S > 8) return w < 16 && S <= 16 && MT <= 2 && nu > 64 ? 12 : w;
         if (MT == 2 && nu < 16) return 8;
         if (w < 16) return 12;
         const int p = passes(16);
