@@ -1,5 +1,5 @@
-// Prefill GEMM (m >= 5 through qk_matmul and grouped launches) for Q8_0 / Q4_K / Q5_K / Q6_K weights: super-blocks dequantized to fp16
-// feeding CDNA4 MFMA (v_mfma_f32_32x32x16_f16), fp32 accumulate.
+// Prefill GEMM (from 17 tokens, and below where qk_few.hip has no plan) for Q8_0 / Q4_K / Q5_K / Q6_K weights:
+// super-blocks dequantized to fp16 feeding CDNA4 MFMA (v_mfma_f32_32x32x16_f16), fp32 accumulate.
 //
 // Replaces the reference's k_gemm_q4k / k_gemm_q6k (qwen_cuda/kernels.cu:307-361, 394, 397-401:
 // 64x64x64 tiles, 2x2 warps of mma.m16n8k16, dequant via dq8h into shared memory) with a design
@@ -22,8 +22,8 @@
 //    weights), so the dequantized weights never travel through LDS.  One barrier per step.
 //  * x is read as fp16 [m][k] where it lies when the caller passes fp16, as the reference's GEMM
 //    takes it (no prepass), also in the xperm layout its decode path feeds for m < 16; fp32 x is
-//    first rounded to fp16 by k_gemm_cvt_x.  Each LDS-DMA of activations moves eight tokens'
-//    16-byte k-pieces (whole 128-byte lines in the plain layout) into B-operand order.
+//    first rounded to fp16 by k_gemm_cvt_x.  Each LDS-DMA of activations moves eight tokens' whole
+//    128-byte lines, eight lanes a line, its 16-byte k-pieces permuted within the line.
 //  * y is fp32 [m][n] row-major like the reference's GEMM output (y[tok*n + row]).
 #include <atomic>
 
@@ -52,11 +52,13 @@ __device__ inline f16v mfma32(const h8& a, const h8& b, const f16v& c) {
 // (qwen_cuda/qwen.cpp:246): fp16 x straight from the caller, fp32 x after k_gemm_cvt_x has rounded
 // it to nearest even into the workspace.  A step's 64 k of one token are one aligned 128-byte line,
 // and one LDS-DMA (64 lanes x 16 bytes) moves eight tokens' lines of a 32-token block: DMA j of the
-// block takes tokens 8j .. 8j + 7, lane i the 16 bytes of token 8j + (i & 7) that hold its k-piece
-// p = 2 (i >> 4) + (((i >> 3) & 1) ^ (j & 1)) (eight halves, k = 8p .. 8p + 7 of the step).  The
-// B operand of chunk c (k 16c .. 16c + 15) for lane l (token t = l & 31, half h = l >> 5) is then at
-// 1024 (t >> 3) + 128 (h ^ ((t >> 3) & 1)) + 16 (t & 7) + 256 c of the block's 4 KiB: the chunk is an
-// immediate offset, and the 16 lanes of each 256-byte LDS cycle read 16 different 16-byte bank groups.
+// block takes tokens 8j .. 8j + 7, eight lanes a line (lanes that each took 16 bytes of another token's
+// line cost a line lookup apiece), lane i the 16 bytes of token t = 8j + (i >> 3) that hold its k-piece
+// p = (i & 7) ^ ((t >> 1) & 7) (eight halves, k = 8p .. 8p + 7 of the step).  The block's 4 KiB then hold
+// token t at 128 t and its piece p at slot p ^ ((t >> 1) & 7) of the line, so that the 16 lanes of each
+// 256-byte LDS cycle read 16 different 16-byte bank groups.  The B operand of chunk c (k 16c .. 16c + 15) for
+// lane l (t = l & 31, half h = l >> 5) is piece 2c + h: offset 128 t + 16 (h ^ ((t >> 1) & 7)) with chunk c's
+// bits flipped in (^ 32 c).
 __global__ __launch_bounds__(256) void k_gemm_cvt_x(const float* __restrict__ x, size_t n8, u4* __restrict__ xh) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += (size_t)gridDim.x * 256) {
         const f4 a = *(const f4*)(x + 8 * i), b = *(const f4*)(x + 8 * i + 4);
@@ -560,9 +562,9 @@ __global__ __launch_bounds__(THREADS) void k_gemm(const GemmMats mats, int nsb_r
         for (int e = 0; e < 16; e++) accs[i][e] = 0.0f;
 
     // activation DMAs: steps 0 .. STAGES - 2 now, step s + STAGES - 1 in region 2 of step s
-    // compute wave w issues DMA j = w of every token block: lane i brings token 8w + (i & 7) (tokens
-    // past m re-read token m - 1; their columns are never stored), k-piece 2 (i >> 4) + (((i >> 3) & 1)
-    // ^ (w & 1)) of each step
+    // compute wave w issues DMA j = w of every token block: lane i brings token 8w + (i >> 3) (tokens
+    // past m re-read token m - 1; their columns are never stored), k-piece (i & 7) ^ ((4 w + (i >> 4)) & 7)
+    // of each step
     // x in the xperm layout (runs of 1024 elements permuted, xperm_pos): element e = 64 T + 8 p of
     // global step T and k-piece p sits at 1024 (T >> 4) + 256 (p & 3) + 64 ((T >> 2) & 3) + 16 (T & 3)
     // + 8 (p >> 2), a 16-byte run like the plain layout's, so a lane keeps its part (256 (p & 3) +
@@ -597,7 +599,9 @@ __global__ __launch_bounds__(THREADS) void k_gemm(const GemmMats mats, int nsb_r
     typename C::Src src[NPL];
     h8 a[2][NPL], b[OWN > 0 ? NTB : 1], bs;
     auto tile_idx = [&](int i) { return 2 * pair_of(i) + u; };
-    // per-lane LDS bases: every step adds its stage offset once, the rest are immediate offsets
+    // per-lane LDS bases: every step adds its stage offset once, the rest are immediate offsets (a chunk's
+    // bits are flipped into the sum: stages start on whole lines, so it stays within the token's)
+    static_assert(L::STAGE % 128 == 0, "stages hold whole activation lines");
     const int xl = xb_lane_off(lane, 0);
     const uint8_t* const rown = sR(0) + (2 * wave * OWN + u) * L::RPIECES * 256 + 16 * r + 8 * h;
     const uint8_t* const rsh = sR(0) + (8 * OWN + u) * L::RPIECES * 256 + 16 * r + 8 * h;
@@ -913,38 +917,55 @@ int launch_plan(const GemmCall& c, const GemmPlan& pl) {
     return -1;
 }
 
+// A call of more than one round of work-groups ends in a round that only part of the CUs share:
+// where it is estimated faster, its whole rounds run as one launch (P = 8) and the rows left over as
+// a second with a plan of their own, whose K-parts fill the CUs.  The estimate here is the plan's with
+// what single calls hide in the ranking: P = 8 rounds at 1.13 of it (72..74 us for 65 at K = 5120), 8 us
+// for the second launch and its sum, partials written and read; and 5 % in its favour.  Measured (us,
+// one launch / two): Q8_0 6144 x 5120 at 2048 tokens 174 / 138, Q4_K 17408 x 5120 389 / 340, Q6_K
+// 17408 x 5120 486 / 437, Q4_K 5120 x 17408 at 640 134 / 121, at 2048 363 / 347; below the line Q4_K 5120 x
+// 17408 at 1024 181 / 186 and at 1500 265 / 277, which stay single.
+constexpr int ROUND_P = 8;
+struct RoundSplit {
+    int rows = 0;  // of the first launch; 0: one launch
+    GemmPlan tail;
+};
+GemmCall rows_of(const GemmCall& c, int row0, int rows, int tile_bytes) {
+    GemmCall part = c;
+    part.n[0] = rows;
+    part.w[0] = c.w[0] + (size_t)(row0 / 16) * tile_bytes;
+    part.y[0] = (float*)c.y[0] + row0;
+    part.ldy = c.n[0];
+    return part;
+}
+template <int TYPE, int NTB>
+RoundSplit whole_rounds(const GemmCall& c, const GemmPlan& one) {
+    constexpr int P = ROUND_P;
+    RoundSplit r;
+    if (c.nz != 1 || c.glu || g_gemm_p || g_gemm_ks) return r;
+    const int mblocks = (c.m + 32 * NTB - 1) / (32 * NTB), px = ((c.n[0] / 16 + 1) / 2 + P - 1) / P;
+    // whole rounds on every XCD: both maps give it px0 / 8 (or px0 mblocks / 8) whole units
+    const int rounds = (int)((long long)px * mblocks / c.cus), px0 = c.cus / XCDS * rounds / mblocks * XCDS;
+    if (rounds < 1 || px0 < 1 || px0 >= px) return r;
+    const int rows = px0 * P * 32;
+    GemmCall b = c;
+    b.n[0] = c.n[0] - rows;
+    const GemmPlan tail = plan_ntb<TYPE, NTB>(b);
+    auto us = [](const GemmPlan& pl) { return pl.p % 4 == 1 ? pl.t : 1.13 * pl.t; };
+    const double two = 1.13 * rounds * (step_us<TYPE, NTB>(P, c.nsb) + 5.0) + us(tail) + 8.0 +
+                       (tail.ks > 1 ? tail.ks * 4.0 * c.m * (double)b.n[0] / 5e6 : 0.0);
+    if (1.05 * two < us(one)) r = {rows, tail};
+    return r;
+}
+
 template <int TYPE, int NTB>
 int launch_ntb(const GemmCall& c) {
     const GemmPlan one = plan_ntb<TYPE, NTB>(c);
     if constexpr (NTB == 4) {
-        // A call of more than one round of work-groups ends in a round that only part of the CUs share:
-        // where it is estimated faster, its whole rounds run as one launch (P = 8) and the rows left over as
-        // a second with a plan of their own, whose K-parts fill the CUs.  The estimate here is the plan's with
-        // what single calls hide in the ranking: P = 8 rounds at 1.13 of it (72..74 us for 65 at K = 5120), 8 us
-        // for the second launch and its sum, partials written and read; and 5 % in its favour.  Measured (us,
-        // one launch / two): Q8_0 6144 x 5120 at 2048 tokens 174 / 138, Q4_K 17408 x 5120 389 / 340, Q6_K
-        // 17408 x 5120 486 / 437, Q4_K 5120 x 17408 at 640 134 / 121, at 2048 363 / 347; below the line Q4_K 5120 x
-        // 17408 at 1024 181 / 186 and at 1500 265 / 277, which stay single.
-        constexpr int P = 8;
-        const int mblocks = (c.m + 32 * NTB - 1) / (32 * NTB), px = ((c.n[0] / 16 + 1) / 2 + P - 1) / P;
-        // whole rounds on every XCD: both maps give it px0 / 8 (or px0 mblocks / 8) whole units
-        const int rounds = (int)((long long)px * mblocks / c.cus), px0 = c.cus / XCDS * rounds / mblocks * XCDS;
-        if (c.nz == 1 && !c.glu && !g_gemm_p && !g_gemm_ks && rounds >= 1 && px0 >= 1 && px0 < px) {
-            const int rows = px0 * P * 32;
-            GemmCall a = c, b = c;
-            a.n[0] = rows;
-            b.n[0] = c.n[0] - rows;
-            b.w[0] = c.w[0] + (size_t)(rows / 16) * c.nsb * Gcfg<TYPE>::GBYTES;
-            b.y[0] = (float*)c.y[0] + rows;
-            a.ldy = b.ldy = c.n[0];
-            const GemmPlan tail = plan_ntb<TYPE, NTB>(b);
-            auto us = [](const GemmPlan& pl) { return pl.p % 4 == 1 ? pl.t : 1.13 * pl.t; };
-            const double two = 1.13 * rounds * (step_us<TYPE, NTB>(P, c.nsb) + 5.0) + us(tail) + 8.0 +
-                               (tail.ks > 1 ? tail.ks * 4.0 * c.m * (double)b.n[0] / 5e6 : 0.0);
-            if (1.05 * two < us(one)) {
-                const int rc = launch_p<TYPE, P, NTB>(a, 1);
-                return rc != 0 ? rc : launch_plan<TYPE, NTB>(b, tail);
-            }
+        if (const RoundSplit r = whole_rounds<TYPE, NTB>(c, one); r.rows) {
+            const int tile = c.nsb * Gcfg<TYPE>::GBYTES;
+            const int rc = launch_p<TYPE, ROUND_P, NTB>(rows_of(c, 0, r.rows, tile), 1);
+            return rc != 0 ? rc : launch_plan<TYPE, NTB>(rows_of(c, r.rows, c.n[0] - r.rows, tile), r.tail);
         }
     }
     return launch_plan<TYPE, NTB>(c, one);
@@ -1042,6 +1063,22 @@ int launch_call(int type, GemmCall& c, int k, const void* x, int xfmt, uint8_t* 
     return -1;
 }
 }  // namespace
+
+int gemm_round_rows(int type, int k, int n, int m, size_t part_cap, int cus) {
+    GemmCall c{};
+    c.nz = 1;
+    c.n[0] = n;
+    c.nsb = k / 256;
+    c.m = m;
+    c.part_cap = part_cap;
+    c.cus = cus;
+    if (m <= 64) return 0;
+    if (type == T_Q4_K) return whole_rounds<T_Q4_K, 4>(c, plan_ntb<T_Q4_K, 4>(c)).rows;
+    if (type == T_Q5_K) return whole_rounds<T_Q5_K, 4>(c, plan_ntb<T_Q5_K, 4>(c)).rows;
+    if (type == T_Q6_K) return whole_rounds<T_Q6_K, 4>(c, plan_ntb<T_Q6_K, 4>(c)).rows;
+    if (type == T_Q8_0) return whole_rounds<T_Q8_0, 4>(c, plan_ntb<T_Q8_0, 4>(c)).rows;
+    return 0;
+}
 
 int launch_gemm(int type, const uint8_t* w, int k, int n, const void* x, int xfmt, int m, uint8_t* ximg, float* y,
                 float* part, size_t part_cap, hipStream_t s) {

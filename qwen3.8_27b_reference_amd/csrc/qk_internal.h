@@ -117,6 +117,9 @@ int launch_gemm_group(int type, const uint8_t* const* ws, const int* ns, float* 
 // part (at least 2 m n floats), then k_glu_sum adds the parts and stores.  -1 when part is too small.
 int launch_gemm_glu(int type, const uint8_t* wg, const uint8_t* wu, int k, int n, const void* x, int xfmt, int m,
                     uint8_t* ximg, void* y, int yfmt, float* part, size_t part_cap, hipStream_t s);
+// Rows of the first launch of a call that runs as whole rounds and a second launch over the rest; 0: one
+// launch.  Plans only (for tests).
+int gemm_round_rows(int type, int k, int n, int m, size_t part_cap, int cus);
 // Few-token GEMM (qk_few.hip, m <= FEW_MAX_M): all tiles of cnt matrices in one launch, `slices` K-slices x `wgs`
 // work-groups of `waves` waves.  y[z]: [slices][m][n[z]] fp32.
 constexpr int FEW_MAX_M = 16;

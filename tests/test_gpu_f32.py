@@ -36,7 +36,9 @@ SHAPES = [(256, 1, 1), (1280, 3, 2), (5120, 48, 4), (768, 5, 5), (256, 17, 9), (
           # a wave per two or four rows (k <= 768, many rows), ragged rows and tokens, one past its longest k
           (256, 4097, 1), (512, 5003, 3), (768, 1027, 16), (256, 2052, 7), (512, 1500, 11), (768, 4099, 1), (1024, 4099, 1),
           # 16 x 16 tiles: at 256 tiles and one past, ragged rows and tokens, on the line of 44 Ki outputs
-          (1280, 4096, 11), (256, 4091, 16), (768, 4097, 13), (2304, 44, 1024), (256, 47, 1013), (5120, 241, 255)]
+          (1280, 4096, 11), (256, 4091, 16), (768, 4097, 13), (2304, 44, 1024), (256, 47, 1013), (5120, 241, 255),
+          # the same on xperm x
+          (1024, 4096, 11), (2048, 3009, 15)]
 
 
 @pytest.mark.parametrize("k,n,m", SHAPES, ids=[f"k{k}n{n}m{m}" for k, n, m in SHAPES])
@@ -93,3 +95,24 @@ def test_f32_tile_sums(qk, dev, n, m):
     ref = xh.astype(np.float64) @ w.view(np.float32).reshape(n, k).astype(np.float64).T
     err = np.linalg.norm(yd.get(np.float32, (m, n)) - ref) / np.linalg.norm(ref)
     assert err < 1.9e-7, err
+
+
+def test_f32_group_on_tiles(qk, oracle, dev):
+    """A group of 44 Ki outputs and more: matrices of different heights on 16 x 16 tiles, one per grid z."""
+    k, m, ns = 1024, 13, (2048, 1031, 512, 7)
+    assert sum(ns) * m >= 44 * 1024 and sum(-(-n // 16) for n in ns) <= 256
+    ws = [_weights(n, k, 60 + n) for n in ns]
+    xh = oracle.normal(SEED_BASE | 0x350, m * k).reshape(m, k).astype(np.float16)
+    bufs = [dev.put(w) for w in ws]
+    Ws = [qk.weight_view(b.ptr, T_F32, k, n, 0) for b, n in zip(bufs, ns)]
+    for fmt, xa in ((F32, xh.astype(np.float32)), (F16, xh), (F16X, _xperm(xh))):
+        xd, ys = dev.put(xa), [dev.empty((m * n + 64) * 4) for n in ns]
+        for y in ys:
+            y.fill_nan()
+        qk.gemv_group_act(Ws, [y.ptr for y in ys], False, xd.ptr, fmt, m, F32, dev.stream())
+        for w, n, yd in zip(ws, ns, ys):
+            y = yd.get(np.float32, (m * n + 64,))
+            assert np.isnan(y[m * n:]).all()
+            ref, mag = oracle.matmul_f64(T_F32, w, k, n, xh.astype(np.float32))
+            e_max, e_norm = rel_errors(y[:m * n].reshape(m, n), ref, mag)
+            assert e_max < TOL and e_norm < TOL, (n, fmt, e_max, e_norm)

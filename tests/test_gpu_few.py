@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from oracle_lib import SEED_BASE, T_Q4_K, T_Q5_K, T_Q6_K, T_Q8_0, rel_errors
+from test_few_plan import _plan
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +79,36 @@ def test_few_group_heights(qk, oracle, dev, m):
         ref, mag = oracle.matmul_f64(T_Q4_K, w, k, n, xh.astype(np.float32))
         e_max, e_norm = rel_errors(y, ref, mag)
         assert e_max <= TOL and e_norm <= TOL, (n, e_max, e_norm)
+
+
+# (type, k, n, m, waves): 128 units and more a work-group, so twelve waves, rings refilled many times and tiles cut
+# between the waves; Q8_0 whose LDS holds eight
+TALL = [(t, 1024, 131088, m, 12) for t in TYPES for m in (8, 13)] + [(T_Q8_0, 4096, 28704, 8, 8)]
+
+
+@pytest.mark.parametrize("typ,k,n,m,waves", TALL, ids=[f"{IDS[TYPES.index(t)]}k{k}m{m}" for t, k, n, m, _ in TALL])
+def test_few_many_units(qk, oracle, dev, typ, k, n, m, waves):
+    """Every row of a tall matrix whose rows repeat every 1040 (65 tiles, no multiple of a work-group's)."""
+    plan, _ = _plan(qk, typ, k, [n], m)
+    units = -(-plan.ntiles // plan.wgs) * -(-plan.nsb // plan.slices)
+    assert plan.waves == waves and units >= 128
+    base = 1040
+    w = oracle.weights(typ, base, k, SEED_BASE | (0x440 + m)).reshape(base, -1)
+    xh = oracle.normal(SEED_BASE | (0x450 + m), m * k).reshape(m, k).astype(np.float16)
+    W = qk.upload(np.ascontiguousarray(np.resize(w, (n, w.shape[1]))).reshape(-1), typ, k, n, 1)
+    ys = []
+    try:
+        for fmt, xa in ((F16, xh), (F16X, _xperm(xh))):
+            xd, yd = dev.put(xa), dev.empty((m * n + 64) * 4)
+            yd.fill_nan()
+            qk.matmul_act(W, xd.ptr, fmt, m, yd.ptr, dev.stream())
+            y = yd.get(np.float32, (m * n + 64,))
+            assert np.isfinite(y[:m * n]).all() and np.isnan(y[m * n:]).all()
+            ys.append(y[:m * n].reshape(m, n))
+    finally:
+        qk.free(W)
+    assert np.array_equal(ys[0].view(np.uint32), ys[1].view(np.uint32))
+    ref, mag = oracle.matmul_f64(typ, w.reshape(-1), k, base, xh.astype(np.float32))
+    rows = np.arange(n) % base
+    e_max, e_norm = rel_errors(ys[0], ref[:, rows], mag[:, rows])
+    assert e_max <= TOL and e_norm <= TOL, (e_max, e_norm)
