@@ -110,8 +110,8 @@ GLU_GEMM = [(T_Q4_K, 5120, 17408, 13), (T_Q4_K, 5120, 2048, 5), (T_Q4_K, 5120, 2
 
 @pytest.mark.parametrize("typ,k,n,m", GLU_GEMM, ids=[f"{IDS[TYPES.index(t)]}-k{k}n{n}m{m}" for t, k, n, m in GLU_GEMM])
 def test_glu_pair_gemm(qk, oracle, dev, typ, k, n, m):
-    """The gate/up pair from five tokens by default: both matrices in one GEMM launch, the K-parts
-    added in order and silu(g) u applied by k_glu_sum (the C3a shape at 13 tokens included).  Held to
+    """The gate/up pair from five tokens by default: both matrices in one launch (the few-token kernel), the
+    K-slices added in order and silu(g) u applied by k_glu_sum (the C3a shape at 13 tokens included).  Held to
     the MFMA path's bar carried through the product, against the f64 oracle fed the fp16-rounded x
     the GEMM multiplies."""
     wg, wu, x, y, plan = _glu(qk, oracle, dev, typ, k, n, m, 0x1000)
@@ -154,7 +154,7 @@ def test_eight_slot_splits_bitwise_equal(qk, oracle, dev, typ, k, n, m):
                                      (T_Q8_0, 3072, 512)], ids=["c1", "c2", "q5k", "q8_0"])
 @pytest.mark.parametrize("m", [5, 8, 9, 13, 15])
 def test_default_route(qk, oracle, dev, typ, k, n, m):
-    """qk_matmul's own route for five to fifteen tokens: the GEMM in one weight pass, held to the MFMA
+    """qk_matmul's own route for five to fifteen tokens: the few-token GEMM in one weight pass, held to the MFMA
     path's bar (5e-3 on both metrics) against the f64 oracle fed the fp16-rounded x the GEMM
     multiplies, and against the unrounded fp32 x.  The same x rounded to fp16 and laid out in the
     reference's xperm decode layout takes the same GEMM through qk_matmul_act: bitwise equal."""

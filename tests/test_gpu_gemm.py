@@ -239,9 +239,9 @@ GROUPS = {
 @pytest.mark.parametrize("m", [9, 13, 15])
 @pytest.mark.parametrize("group", sorted(GROUPS))
 def test_gemm_group(qk, oracle, dev, group, m):
-    """Shared-x launches (qk_gemv_group) from nine tokens: each run of one type in one GEMM launch, a
-    matrix per grid z (the decode step's {qkv, gate_z, alpha, beta} and {q, k, v} at K=5120 and their
-    real heights; runs split by type; 48- and 80-row matrices leave partial tile pairs).  Every output
+    """Shared-x launches (qk_gemv_group) from nine tokens: each run of one type in one launch of the few-token
+    kernel (the decode step's {qkv, gate_z, alpha, beta} and {q, k, v} at K=5120 and their real heights; runs
+    split by type; tests/test_gpu_gemm_multi.py runs the GEMM's own form, a matrix per grid z).  Every output
     against the f64 oracle fed the fp16-rounded x, at the MFMA path's bar (strided rows of the large
     matrices)."""
     k = 5120 if group != "mixed" else 3072
@@ -274,7 +274,7 @@ def test_gemm_group(qk, oracle, dev, group, m):
 
 def test_gemm_group_with_f32(qk, oracle, dev):
     """{qkv, gate_z, alpha, beta} with F32 alpha / beta (the GGUF's own types) at 13 tokens: the Q4_K
-    run on the GEMM, the F32 matrices on their own kernel (fp32, exact products)."""
+    run on the few-token GEMM, the F32 matrices on their own kernel (fp32, exact products)."""
     k, m = 1024, 13
     rng = np.random.default_rng(11)
     wq = [oracle.weights(T_Q4_K, n, k, SEED_BASE | (0xBA + i)) for i, n in enumerate((320, 192))]

@@ -118,7 +118,7 @@ def test_gemv_stream_split(qk, oracle, dev, typ, waves):
 
 
 # (13056, 2048): three K-slices (a slice-tree node without a sibling), ranges straddling slices and
-# groups; (19200, 1600): five slices for Q6_K, three for Q4_K
+# groups; (19200, 1600): five
 FUSED_SHAPES = [(256, 16), (512, 48), (1024, 64), (5120, 256), (17408, 1024), (6144, 5120), (13056, 2048),
                 (19200, 1600)]
 
