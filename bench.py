@@ -4,9 +4,9 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload c2] [--no-cpu] [--no-extras]
 
 A step is one pass of the hot path over one batch of synthetic input: one qk_matmul /
-qk_gemv_group call through the C ABI (M=1..8: the int8 GEMV kernel alone, x converted inside;
-M>=16: the GEMM kernel on fp16 x as the reference's GEMM takes it, or with fp32 x a rounding pass
-first), or for c5 the 257 grouped launches of one decode step.  The K timed steps are captured
+qk_gemv_group call through the C ABI (M=1..4: the int8 GEMV kernel alone, x converted inside; M=5..16:
+the few-token GEMM; above: the GEMM kernel; both on fp16 x as the reference's GEMM takes it, or with
+fp32 x a rounding pass first), or for c5 the 257 grouped launches of one decode step.  The K timed steps are captured
 once into a HIP graph, replayed untimed until at least 0.2 s of GPU work has run and two replays
 agree within 1 % (the steady state of a stream of calls), then replayed once more, timed; every step uses a different weight copy from a ring of copies totalling
 >= 512 MiB, so the 256 MiB Infinity Cache cannot serve repeats.  Inputs are resident in HBM before
@@ -75,25 +75,25 @@ CONFIGS = {
     "q6k_gate": dict(desc="Q6_K GEMV M=1 K=5120 N=17408", kind="gemv", type=T_Q6_K, K=5120, N=17408, M=1, cid=13),
     # batched decode below 16 tokens (the reference's GEMV for every T < 16 reads the weights once per
     # eight tokens, NT = 8 at qwen_cuda/kernels.cu:11, qwen.cpp:240-247): one pass here at M=8 and M=13
-    "c1_m8": dict(desc="Q4_K matmul M=8 K=5120 N=17408 (C1 shape; qk_matmul's route from 5 tokens: the GEMM, one "
+    "c1_m8": dict(desc="Q4_K matmul M=8 K=5120 N=17408 (C1 shape; qk_matmul's route for 5..16 tokens: the few-token GEMM, one "
                        "weight pass)", kind="gemv", type=T_Q4_K,
                   K=5120, N=17408, M=8, cid=14),
-    "c1_m13": dict(desc="Q4_K matmul M=13 K=5120 N=17408 (C1 shape; qk_matmul's route from 5 tokens: the GEMM, one "
+    "c1_m13": dict(desc="Q4_K matmul M=13 K=5120 N=17408 (C1 shape; qk_matmul's route for 5..16 tokens: the few-token GEMM, one "
                         "weight pass)", kind="gemv", type=T_Q4_K, K=5120, N=17408, M=13, cid=15),
-    "c2_m8": dict(desc="Q6_K matmul M=8 K=17408 N=5120 (C2 shape; qk_matmul's route from 5 tokens: the GEMM, one "
+    "c2_m8": dict(desc="Q6_K matmul M=8 K=17408 N=5120 (C2 shape; qk_matmul's route for 5..16 tokens: the few-token GEMM, one "
                        "weight pass)", kind="gemv", type=T_Q6_K,
                   K=17408, N=5120, M=8, cid=16),
-    "c2_m13": dict(desc="Q6_K matmul M=13 K=17408 N=5120 (C2 shape; qk_matmul's route from 5 tokens: the GEMM, one "
+    "c2_m13": dict(desc="Q6_K matmul M=13 K=17408 N=5120 (C2 shape; qk_matmul's route for 5..16 tokens: the few-token GEMM, one "
                         "weight pass)", kind="gemv", type=T_Q6_K, K=17408, N=5120, M=13, cid=17),
     # the same 13-token calls on the activations the reference's forward feeds for T < 16: fp16 in its
     # xperm layout (qwen_cuda/qwen.cpp:234), read by the GEMM where they lie
-    "c1_m13x": dict(desc="Q4_K matmul M=13 K=5120 N=17408 (C1 shape, fp16 xperm x: the GEMM, one weight pass)",
+    "c1_m13x": dict(desc="Q4_K matmul M=13 K=5120 N=17408 (C1 shape, fp16 xperm x: the few-token GEMM, one weight pass)",
                     kind="gemv", type=T_Q4_K, K=5120, N=17408, M=13, cid=18, xf16=True, xperm=True),
-    "c2_m13x": dict(desc="Q6_K matmul M=13 K=17408 N=5120 (C2 shape, fp16 xperm x: the GEMM, one weight pass)",
+    "c2_m13x": dict(desc="Q6_K matmul M=13 K=17408 N=5120 (C2 shape, fp16 xperm x: the few-token GEMM, one weight pass)",
                     kind="gemv", type=T_Q6_K, K=17408, N=5120, M=13, cid=19, xf16=True, xperm=True),
     # the decode FFN's gate/up launch at 13 tokens as the reference's forward issues it: fp16 xperm x in,
-    # fp16 silu(g) u out at xperm(row) (qwen_cuda/qwen.cpp:264, kernels.cu:419-426); both matrices on the GEMM
-    "c3a_m13x": dict(desc="Q4_K gate+up GLU M=13 K=5120 N=17408x2 (C3a shape, fp16 xperm x and output: the GEMM, "
+    # fp16 silu(g) u out at xperm(row) (qwen_cuda/qwen.cpp:264, kernels.cu:419-426); both matrices on the few-token GEMM
+    "c3a_m13x": dict(desc="Q4_K gate+up GLU M=13 K=5120 N=17408x2 (C3a shape, fp16 xperm x and output: the few-token GEMM, "
                           "one weight pass)", kind="glu", type=T_Q4_K, K=5120, N=17408, M=13, cid=22, xf16=True,
                      xperm=True, yf16=True),
     "q5k_m512": dict(desc="Q5_K prefill GEMM M=512 K=17408 N=5120 (fp16 x)", kind="gemm", type=T_Q5_K, K=17408,
@@ -116,9 +116,10 @@ SWEEP_LAYERS = 64
 # The reference's own published GEMV bandwidth for the same shapes on an RTX 6000D
 # (notes/parallel_decode_experiments.md:111-116 of the reference).
 REF_PUBLISHED_GBS = {"c1": 1192.0, "c2": 1214.0, "q4k_down": 1188.0, "q6k_gate": 1205.0}
-KERNEL_SINGLE = "k_gemv1"  # M = 1..8 per launch: one kernel, x converted inside
-GEMM_ROUTE_M = 5  # qk_matmul sends m >= 5 to the GEMM (include/qk.h)
+KERNEL_SINGLE = "k_gemv1"  # M = 1..4 here: one kernel, x converted inside
+GEMM_ROUTE_M = 5  # qk_matmul sends m >= 5 to the GEMM (include/qk.h), up to 16 tokens in its few-token form
 KERNEL_GEMM = "k_gemm"
+KERNEL_FEW = "k_few"
 KERNEL_EMBED = "k_embed"
 
 
@@ -670,8 +671,8 @@ def main():
                  "gbs": round(gbs, 1), "us_per_call": round(ms * 1e3, 2), "roofline": rf}
         else:
             cfg = CONFIGS[name]
-            routed = cfg["kind"] in ("gemv", "glu") and cfg["M"] >= GEMM_ROUTE_M  # the GEMM route
-            kernel = KERNEL_GEMM if cfg["kind"] == "gemm" or routed else KERNEL_SINGLE
+            routed = cfg["kind"] in ("gemv", "glu") and cfg["M"] >= GEMM_ROUTE_M  # the few-token GEMM
+            kernel = KERNEL_GEMM if cfg["kind"] == "gemm" else KERNEL_FEW if routed else KERNEL_SINGLE
             rf = roofline(name, cfg, r["ms_per_step"], r["bytes_per_step"], kernel)
             d = {"desc": cfg["desc"]}
             if cfg["kind"] == "gemm":
@@ -683,17 +684,16 @@ def main():
                 rf["timed_unit"] = ("one call = one k_gemv1 launch (x converted into the int8 image inside)"
                                     if not routed else
                                     "one qk_gemv_group_act call of the gate/up pair on fp16 xperm x, which it "
-                                    "sends to the GEMM from 5 tokens: both matrices in one k_gemm launch, then "
-                                    "k_glu_sum adds the K-parts and writes fp16 silu(g) u at xperm(row); one "
+                                    "sends to the few-token GEMM: both matrices in one k_few launch, then "
+                                    "k_glu_sum adds the K-slices and writes fp16 silu(g) u at xperm(row); one "
                                     "weight pass"
                                     if cfg["kind"] == "glu" else
                                     "one qk_matmul_act call on fp16 x in the xperm layout, which it sends to the "
-                                    "GEMM from 5 tokens: k_gemm reading x where it lies, in work-groups of one "
-                                    "32-token block (+ the split-K sum), one weight pass"
+                                    "few-token GEMM: k_few reading x where it lies (+ the split-K sum), one weight "
+                                    "pass"
                                     if cfg.get("xperm") else
-                                    "one qk_matmul call, which sends m >= 5 to the GEMM: k_gemm_cvt_x (fp32 x "
-                                    "rounded to fp16) + k_gemm in work-groups of one 32-token block (+ the split-K "
-                                    "sum), one weight pass")
+                                    "one qk_matmul call, which sends 5..16 tokens to the few-token GEMM: k_gemm_cvt_x "
+                                    "(fp32 x rounded to fp16) + k_few (+ the split-K sum), one weight pass")
             if name in REF_PUBLISHED_GBS:
                 d["ref_rtx6000d_gbs"] = REF_PUBLISHED_GBS[name]
             if "ceiling" in r:

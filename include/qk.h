@@ -132,11 +132,15 @@ int qk_embed(const qk_weight* table, const int32_t* tokens, const uint8_t* mask,
              qk_stream_t stream);
 
 /* y[m][n] = sum_k W[n][k] * x[m][k]; x fp32 [m][k], y fp32 [m][n], both 16-byte aligned.
- * m <= 4 runs the fused-dequant MFMA GEMV, m >= 5 the LDS-dequant MFMA GEMM (qwen_cuda/qwen.cpp:240-247
- * matmul, which runs its GEMV below 16 tokens on fp16 x; CPU Ops::matmul qwen_cpu/ops.h:54-76): from
- * five tokens the GEMV's eight-token form is compute-bound (and needs a second weight pass from nine)
- * while the GEMM, one 32-token block per work-group, reads the weights once at the memory system's
- * pace (the gemm_min_m knob moves the boundary).  The GEMV path
+ * m <= 4 runs the fused-dequant MFMA GEMV, m >= 5 an MFMA GEMM on fp16 operands (qwen_cuda/qwen.cpp:240-247
+ * matmul, which runs its GEMV below 16 tokens on fp16 x; CPU Ops::matmul qwen_cpu/ops.h:54-76): from five
+ * tokens the GEMV's eight-token form is compute-bound (and needs a second weight pass from nine) while the
+ * GEMM reads the weights once at the memory system's pace (the gemm_min_m knob moves the boundary).  5..16
+ * tokens run on its few-token form, which streams the weights like the GEMV does beside a slice of x in LDS,
+ * wherever that has a plan; the other calls on the LDS-dequant form in blocks of 32, 64 or 128 tokens, calls of
+ * several rounds of work-groups in two launches where that is estimated faster.  The order of a result's fp32
+ * sums follows the plan, which depends on m and on the matrices that share the launch (F32 matrices
+ * included): a token's last bits may differ with them, the same call gives the same bits.  The GEMV path
  * (int8 MFMA kernel) carries each token's x per 256-element super-block as three int8 parts with
  * fp32 scales, every element within max|x| / 16387064 of its value, for any finite fp32 x (a
  * super-block below 2^-100 is converted from x * 2^100 and scaled back); a NaN or inf in x makes
@@ -161,8 +165,8 @@ int qk_matmul_noalloc(const qk_weight* w, const float* x, int32_t m, float* y, q
 
 /* qk_matmul with x in format xfmt (QK_ACT_*): the reference's matmul(w, x, T, y) with fp16 x
  * (qwen_cuda/qwen.cpp:240-247).  QK_ACT_F16_XPERM needs m < 16 (as in the reference) and k % 1024 == 0.
- * The routing is qk_matmul's for every format: m <= 4 on the GEMV, m >= 5 on the GEMM, which reads
- * fp16 x, plain or xperm, where it lies (no rounding, no copy).  y is fp32 [m][n]. */
+ * The routing is qk_matmul's for every format: m <= 4 on the GEMV, m >= 5 on the GEMM in either form, which
+ * reads fp16 x, plain or xperm, where it lies (no rounding, no copy).  y is fp32 [m][n]. */
 int qk_matmul_act(const qk_weight* w, const void* x, uint32_t xfmt, int32_t m, float* y, qk_stream_t stream);
 
 /* Grouped GEMV for m < 16 (qwen_cuda/qwen.cpp:220-238 gemv, MmGroup kernels.cu:403-438): `cnt`
@@ -170,7 +174,7 @@ int qk_matmul_act(const qk_weight* w, const void* x, uint32_t xfmt, int32_t m, f
  * ws[0]/ws[1] are gate/up with equal n and ys[0][m][n] = silu(gate x) * (up x) in fp32.  A quantized
  * gate/up pair, and each run of one quantized type in a group, of five or more tokens run on the GEMM
  * (a run's matrices in one launch, one weight pass; fp16 operands, the GEMM's bar); fewer tokens on
- * the GEMV, F32 matrices on their own kernel. */
+ * the GEMV, a run of F32 matrices in one launch of their own kernels. */
 int qk_gemv_group(const qk_weight* const* ws, float* const* ys, int32_t cnt, int32_t glu, const float* x, int32_t m,
                   qk_stream_t stream);
 
@@ -220,7 +224,8 @@ int qk_gemv_plan(const qk_weight* const* ws, int32_t cnt, int32_t glu, int32_t m
  * carries, 8 (default: one weight pass per eight tokens) or 4 (m = 5..8 as four tokens and the rest)),
  * "gemm_min_m" (the smallest m qk_matmul and qk_matmul_act route to the GEMM, and qk_gemv_group(_act)
  * a gate/up pair or a group; 2..16, 0 restores the default 5), "gemm_ksplit" (GEMM K-parts, 1..16,
- * partials added in part order by a second kernel; 0 restores the plan), "gemm_pairs" (16-row tile pairs per GEMM work-group: 2, 3, 4, 5, 8 or 9;
+ * partials added in part order by a second kernel; 0 restores the plan), "gemm_pairs" (16-row tile pairs per
+ * GEMM work-group: 2, 3, 4, 5, 8 or 9; either of the two sends calls of 5..16 tokens to the LDS-dequant form;
  * 0 restores the built-in plan) or "gemm_map" (1 = each XCD serves one token block where 2, 4 or 8
  * token blocks divide the XCDs, the default; 0 = the (K-part, pair group) units dealt densely over the
  * XCDs, each with its token blocks on one XCD, which every call with one token block or another count

@@ -33,8 +33,8 @@ constexpr size_t WS_KPART_BYTES = 128ull << 20;  // GEMM split-K partials
 // layout when its forward sets G_xperm; xperm x is accepted for m < GEMM_MIN_M only, as there.
 // From GEMM_ROUTE_M tokens qk_matmul(_act), a group's runs of one type and a gate/up pair take the
 // GEMM instead, any activation format: the int8 GEMV carries eight tokens per launch (two weight
-// passes from nine) and its eight-token form is compute-bound, while the GEMM in work-groups of one
-// 32-token block reads the weights once.  Measured on MI355X (us per call, fp16 xperm x, GEMV
+// passes from nine) and its eight-token form is compute-bound, while the GEMM reads the weights once.
+// Measured on MI355X, before 5..16 tokens had a form of their own (qk_few.hip) (us per call, fp16 xperm x, GEMV
 // against GEMM): at five tokens K=17408 N=5120 Q4_K 29.4 / 22.6, Q6_K 38.0 / 36.4, Q5_K 32.4 / 32.8;
 // K=5120 N=17408 Q4_K 24.2 / 20.3; the output projection 487 / 257; the gate/up pair 46.4 / 32.4;
 // at four tokens the GEMV wins (the pair 25.9 / 32.0).
